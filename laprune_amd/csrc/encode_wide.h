@@ -67,7 +67,7 @@ __device__ __forceinline__ constexpr int wide_dim(int s, int e, int h) {
 }
 
 __device__ __forceinline__ float wide_f16_flushed(float x) {
-  const float y = (float)(_Float16)x;
+  const float y = h2f(f2h(x));
   return fabsf(y) < 0x1p-14f ? 0.f : y;
 }
 
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void encode_prep_wide(const float* __restrict_
     wh8_t v;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      v[e] = (_Float16)(cbm[(int64_t)k * D + wide_dim<D>(ks, e, l >> 5)] * sc);
+      v[e] = __builtin_bit_cast(_Float16, f2h(cbm[(int64_t)k * D + wide_dim<D>(ks, e, l >> 5)] * sc));
     out[i] = __builtin_bit_cast(uint4, v);
   }
   uint2* hp = reinterpret_cast<uint2*>(out + nf);
@@ -147,9 +147,8 @@ __global__ __launch_bounds__(256) void encode_prep_wide(const float* __restrict_
     wh4_t v = {};
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
-      const _Float16 p = (_Float16)x;
-      v[e] = p;
-      x = x - (float)p;
+      v[e] = __builtin_bit_cast(_Float16, f2h(x));
+      x = x - (float)v[e];
     }
     hp[i] = __builtin_bit_cast(uint2, v);
   }
