@@ -18,9 +18,9 @@
 //
 // lap_encode_prepare builds, once per codebook: Ct[m][d][k] (the codebook
 // transposed so that lane-contiguous k is memory-contiguous) and cn[m][k].
-// lap_encode_greedy: one wave per row; lane l owns entries k = 4l..4l+3 and
-// keeps their 16 chain sums in registers while d streams through; the row's
-// residual lives in LDS and is read as a broadcast.
+// encode_greedy_kernel (the VALU form): one wave per row; lane l owns entries
+// k = 4l..4l+3 and keeps their 16 chain sums in registers while d streams
+// through; the row's residual lives in LDS and is read as a broadcast.
 #include "common.h"
 
 #include <algorithm>
@@ -48,10 +48,9 @@ struct Prep {
   float* ct;       // [M][D][K]
   float* cn;       // [M][K]
   float* scn;      // [M][K] sqrtf(cn)
-  uint16_t* frag;  // bf16 MFMA B fragments [M][K/16][D/16][64 lanes][4] (K % 16 == 0)
-  uint16_t* frag4; // 4x4x4 B operands [M][ceil(K/64)][D/8][64 lanes][8] (K % 16 == 0)
-  float4* c4;      // [M][D/4][K] float4: entry k's d = 4q .. 4q+3 (the exact kernel's rows)
-  uint4* wide;     // fp16 fragments of the prompt-sized encode (encode_wide.h)
+  uint16_t* frag;  // bf16 MFMA B fragments [M][K/16][D/16][64 lanes][4] (D = 256)
+  float4* c4;      // [M][D/4][K] float4: entry k's d = 4q .. 4q+3 (the exact kernel's, D = 64)
+  uint4* wide;     // fp16 fragments of the wide and split kernels (encode_wide.h)
   WideStage* wstage;  // [M] its per-stage constants
   size_t bytes;
 };
@@ -70,11 +69,9 @@ Prep carve_prep(void* base, int M, int K, int D) {
   p.scn = reinterpret_cast<float*>(b ? b + off : nullptr);
   off = align_up(off + (size_t)M * K * 4, 256);
   p.frag = reinterpret_cast<uint16_t*>(b ? b + off : nullptr);
-  if (K % 16 == 0) off = align_up(off + (size_t)M * K * D * 2, 256);
-  p.frag4 = reinterpret_cast<uint16_t*>(b ? b + off : nullptr);
-  if (K % 16 == 0) off = align_up(off + (size_t)M * ((K + 63) / 64) * 64 * D * 2, 256);
+  if (K % 16 == 0 && D == 256) off = align_up(off + (size_t)M * K * D * 2, 256);
   p.c4 = reinterpret_cast<float4*>(b ? b + off : nullptr);
-  off = align_up(off + (size_t)M * K * D * 4, 256);
+  if (D == 64) off = align_up(off + (size_t)M * K * D * 4, 256);
   p.wide = reinterpret_cast<uint4*>(b ? b + off : nullptr);
   if (wide_serves(K, D)) off = align_up(off + (size_t)M * wide_stage_uint4(K, D) * 16, 256);
   p.wstage = reinterpret_cast<WideStage*>(b ? b + off : nullptr);
@@ -157,24 +154,6 @@ __global__ __launch_bounds__(256) void encode_prep_c4(const float* __restrict__ 
     const int q = (int)(mq % Q), m = (int)(mq / Q);
     c4[i] = *reinterpret_cast<const float4*>(cb + ((int64_t)m * K + k) * D + 4 * q);
   }
-}
-
-__global__ __launch_bounds__(256) void encode_prep_norms(const float* __restrict__ cb, int M,
-                                                         int K, int D, float* __restrict__ cn,
-                                                         float* __restrict__ scn) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= M * K) return;
-  const float* row = cb + (int64_t)i * D;
-  const int L = D / 16;
-  float s[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    float a = 0.f;
-    for (int t = 0; t < L; ++t) a = __builtin_fmaf(row[j * L + t], row[j * L + t], a);
-    s[j] = a;
-  }
-  cn[i] = fold16(s);
-  scn[i] = sqrtf(cn[i]);
 }
 
 // dot16(r, r) over a row held in LDS: lanes 0..15 each run one chain, the
@@ -324,28 +303,6 @@ __global__ __launch_bounds__(256) void encode_prep_frag(const float* __restrict_
   for (int e = 0; e < 4; ++e) dst[e] = f2bf(src[e]);
 }
 
-// One thread per (m, quarter q, step pair p, lane l): the eight bf16 of
-// C[m][64q + l][8p .. 8p+7] (zeros past K), the B operands of two 4x4x4 steps.
-__global__ __launch_bounds__(256) void encode_prep_frag4(const float* __restrict__ cb, int M,
-                                                         int K, int D,
-                                                         uint16_t* __restrict__ frag4) {
-  const int NQ = (K + 63) / 64, NP = D / 8;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t total = (int64_t)M * NQ * NP * 64;
-  if (i >= total) return;
-  const int l = (int)(i % 64);
-  int64_t q = i / 64;
-  const int pp = (int)(q % NP);
-  q /= NP;
-  const int qq = (int)(q % NQ);
-  const int m = (int)(q / NQ);
-  const int k = qq * 64 + l;
-  uint16_t* dst = frag4 + i * 8;
-  const float* src = cb + ((int64_t)m * K + k) * D + 8 * pp;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) dst[e] = k < K ? f2bf(src[e]) : (uint16_t)0;
-}
-
 // Cross-lane moves within a row of 16 lanes (DPP, no LDS round trip).
 // row_shl:n gives lane i the value of lane i + n of its row (0 past the end).
 template <int CTRL>
@@ -366,6 +323,23 @@ __device__ __forceinline__ float row_fold16(float a) {
   a = a + dpp_f<0x121>(a);  // row_ror:1
   return a;
 }
+// cn = dot16(C, C) per entry, sixteen lanes each (lane j: chain j).
+__global__ __launch_bounds__(256) void encode_prep_norms(const float* __restrict__ cb, int M,
+                                                         int K, int D, float* __restrict__ cn,
+                                                         float* __restrict__ scn) {
+  const int i = blockIdx.x * 16 + (threadIdx.x >> 4), j = threadIdx.x & 15;
+  const bool own = i < M * K;
+  const int L = D / 16;
+  const float* c = cb + (int64_t)(own ? i : 0) * D + j * L;
+  float a = 0.f;
+  for (int t = 0; t < L; ++t) a = __builtin_fmaf(c[t], c[t], a);
+  a = row_fold16(a);
+  if (own && j == 0) {
+    cn[i] = a;
+    scn[i] = sqrtf(a);
+  }
+}
+
 // Minimum over the 16 lanes of a row, in every lane (row_ror rotations).
 __device__ __forceinline__ float row_min16(float a) {
   a = fminf(a, dpp_f<0x128>(a));  // row_ror:8
@@ -710,307 +684,24 @@ __global__ __launch_bounds__(EncCfg<D>::THREADS) void encode_mfma_kernel(
     rnorm[row0 + tid] = sqrtf(s.rn[tid]);
 }
 
-// ------------------------------------------ four rows per workgroup (flushes)
-// The stage of enc_stage for 4 rows, so that a decode flush (8 KV heads x 64
-// tokens = 512 rows) spreads over 128 CUs instead of 32.  The stage chain is
-// latency-bound: a 16-row workgroup has one wave per SIMD, each running 16
-// rows' bound arithmetic, list building and recheck back to back.  Here the
-// coarse dots come from v_mfma_f32_4x4x4bf16_1k (16 blocks of 4x4x4); in
-// block b (lanes 4b .. 4b+3)
-//     D[lane l][v] = sum_k A[lane 4b+v][k] * B[lane l][k]
-// over the four bf16 k terms of a register.  With lane l supplying residual
-// row l % 4 as A and codebook entry 64w + l (wave w) as B, lane l ends with the
-// dots of its entry with all four rows.  The error bound of the 16-row kernel
-// holds as it stands: it covers any fp32 accumulation order of the D exact
-// bf16 products.  After one barrier wave v owns row v: its survivors are four
-// wave-uniform ballots over the row's 256 lower bounds, rechecked four at a
-// time (one candidate per 16-lane group, dot16 chain j in lane j), and the
-// group holding the winner updates the row's residual.  B operands come from
-// the 16x16x16 fragment layout of the prep: entry k's 4 bf16 at d = 4s are
-// fragment lane (k % 16) + 16 (s % 4) of tile k / 16, k-step s / 4, i.e.
-// 16 s uint2 past its step-0 slot.
-constexpr int kR4 = 4;
 // Codes of the first kCodeStage stages are kept in LDS and stored once at
 // the end: a global store inside the stage loop would make the next stage's
 // wait for its operands also wait for the store's acknowledgement.
 constexpr int kCodeStage = 64;
 
-template <int D>
-struct Enc4Shared {
-  float r[kR4][D];
-  uint16_t rb[kR4][D + 8];  // bf16(r); the pitch puts the four rows in different banks
-  float rn[kR4];
-  float2 gb[kR4][256];      // per row, per entry: (lower, upper) bound of the coarse distance
-  uint8_t code[kR4][kCodeStage];  // the rows' codes, written out after the last stage
-};
-
-template <int D>
-struct Enc4Stage {
-  uint4 b[D / 8];  // B operands of steps 2p (x, y) and 2p + 1 (z, w)
-  float cn, scn;
-};
-
-// Stage m's operands of lane l of wave q: entry 64q + l (quarters past K load
-// the last quarter, results ignored), one coalesced 16-byte load per step pair.
-template <int D>
-__device__ __forceinline__ void enc4_load_stage(Enc4Stage<D>& st, const uint4* __restrict__ frag4,
-                                                const float* __restrict__ cn,
-                                                const float* __restrict__ scn, int m, int NQ,
-                                                int K, int qc, int kc, int lane) {
-  const uint4* f = frag4 + (((int64_t)m * NQ + qc) * (D / 8)) * 64 + lane;
-#pragma unroll
-  for (int pp = 0; pp < D / 8; ++pp) st.b[pp] = f[64 * pp];
-  st.cn = cn[(int64_t)m * K + kc];
-  st.scn = scn[(int64_t)m * K + kc];
-}
-
-// Minimum over the 64 lanes of a wave (wave-uniform).
-__device__ __forceinline__ float wave_min64(float a) {
-  a = row_min16(a);
-  const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 0));
-  const float a1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 16));
-  const float a2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 32));
-  const float a3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 48));
-  return fminf(fminf(a0, a1), fminf(a2, a3));
-}
-
-// Lowest set bit of the 256-bit mask m[0..3] (wave-uniform), cleared; -1 if empty.
-__device__ __forceinline__ int pop_lowest(uint64_t& m0, uint64_t& m1, uint64_t& m2, uint64_t& m3) {
-  if (m0) { const int b = __builtin_ctzll(m0); m0 &= m0 - 1; return b; }
-  if (m1) { const int b = __builtin_ctzll(m1); m1 &= m1 - 1; return 64 + b; }
-  if (m2) { const int b = __builtin_ctzll(m2); m2 &= m2 - 1; return 128 + b; }
-  if (m3) { const int b = __builtin_ctzll(m3); m3 &= m3 - 1; return 192 + b; }
-  return -1;
-}
-
-// Pull slice (block / 8) % 16 of codebook m (fp32) into L2 ahead of the exact
-// recheck: the workgroups of one XCD (block ids equal mod 8) take different
-// slices.  One word per 32 bytes; consumed a stage later through a sink.
-template <int D>
-__device__ __forceinline__ uint32_t enc4_prefetch_l2(const float* __restrict__ cb, int m, int K,
-                                                     int tid) {
-  const int64_t words = (int64_t)K * D;
-  const int64_t slice = (words + 15) / 16;
-  const int64_t stride = slice / 256 > 8 ? slice / 256 : 8;
-  int64_t w = ((blockIdx.x >> 3) & 15) * slice + (int64_t)tid * stride;
-  w = w < words - 1 ? w : words - 1;
-  return __builtin_bit_cast(uint32_t, cb[(int64_t)m * words + w]);
-}
-
-template <int D>
-__device__ __forceinline__ void enc4_stage(Enc4Shared<D>& s, const Enc4Stage<D>& st,
-                                           const float* __restrict__ cb,
-                                           const float* __restrict__ cn, int m, int K, int row0,
-                                           int N, const RowMap& rm, bool own, int k, int wave,
-                                           int lane) {
-  constexpr int S4 = D / 4, L = D / 16;
-  // ---- coarse pass: lane l, entry k = 64 wave + l, all four rows
-  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  {
-    const uint16_t* ar = s.rb[lane & 3];
-#pragma unroll
-    for (int t = 0; t < S4; t += 2) {
-      const uint4 aa = *reinterpret_cast<const uint4*>(ar + 4 * t);
-      const uint4 bb = st.b[t / 2];
-      acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
-          __builtin_bit_cast(bf16x4_t, make_uint2(aa.x, aa.y)),
-          __builtin_bit_cast(bf16x4_t, make_uint2(bb.x, bb.y)), acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
-          __builtin_bit_cast(bf16x4_t, make_uint2(aa.z, aa.w)),
-          __builtin_bit_cast(bf16x4_t, make_uint2(bb.z, bb.w)), acc1, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < kR4; ++v) {
-    const float rn = s.rn[v];
-    const float srn = __builtin_amdgcn_sqrtf(rn);
-    const float A = rn + st.cn;
-    const float dm = acc0[v] + acc1[v];
-    const float g = A - 2.0f * dm;
-    const float eps = 0x1.02p-6f * (srn * st.scn) + 0x1p-21f * (fabsf(A) + 2.0f * fabsf(dm)) +
-                      0x1p-116f * (1.0f + srn + st.scn);
-    s.gb[v][k] = own ? make_float2(g - eps, g + eps) : make_float2(INFINITY, INFINITY);
-  }
-  lds_barrier();
-
-  // ---- exact recheck of row v = wave: U = least upper bound over the row
-  const int v = wave, j = lane & 15, grp = lane >> 4;
-  const float2 b0 = s.gb[v][lane], b1 = s.gb[v][64 + lane];
-  const float2 b2 = s.gb[v][128 + lane], b3 = s.gb[v][192 + lane];
-  const float U = wave_min64(fminf(fminf(b0.y, b1.y), fminf(b2.y, b3.y)));
-  uint64_t mk0 = __ballot(lane < K && !(b0.x > U));
-  uint64_t mk1 = __ballot(64 + lane < K && !(b1.x > U));
-  uint64_t mk2 = __ballot(128 + lane < K && !(b2.x > U));
-  uint64_t mk3 = __ballot(192 + lane < K && !(b3.x > U));
-  float rc[L];
-#pragma unroll
-  for (int t = 0; t < L; t += 4) {
-    const float4 x = *reinterpret_cast<const float4*>(&s.r[v][j * L + t]);
-    rc[t] = x.x;
-    rc[t + 1] = x.y;
-    rc[t + 2] = x.z;
-    rc[t + 3] = x.w;
-  }
-  const float rn = s.rn[v];
-  float bc[L];
-#pragma unroll
-  for (int t = 0; t < L; ++t) bc[t] = 0.f;
-  float best = 0.f;
-  int bk = -1;
-  // Batches of four survivors, one per group, lowest entries first.  Ties go
-  // to the lowest entry; NaN and +inf never win.
-  while (mk0 | mk1 | mk2 | mk3) {
-    const int q0 = pop_lowest(mk0, mk1, mk2, mk3);
-    const int q1 = pop_lowest(mk0, mk1, mk2, mk3);
-    const int q2 = pop_lowest(mk0, mk1, mk2, mk3);
-    const int q3 = pop_lowest(mk0, mk1, mk2, mk3);
-    const int kq = grp == 0 ? q0 : grp == 1 ? q1 : grp == 2 ? q2 : q3;
-    if (kq >= 0) {
-      const float* cr = cb + ((int64_t)m * K + kq) * D + j * L;
-      float c[L];
-#pragma unroll
-      for (int t = 0; t < L; t += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(cr + t);
-        c[t] = x.x;
-        c[t + 1] = x.y;
-        c[t + 2] = x.z;
-        c[t + 3] = x.w;
-      }
-      const float cnk = cn[(int64_t)m * K + kq];
-      float dot = 0.f;
-#pragma unroll
-      for (int t = 0; t < L; ++t) dot = __builtin_fmaf(rc[t], c[t], dot);
-      dot = row_fold16(dot);
-      const float E = (rn + cnk) - 2.0f * dot;
-      if (!(E != E) && E != INFINITY && (bk < 0 || E < best || (E == best && kq < bk))) {
-        best = E;
-        bk = kq;
-#pragma unroll
-        for (int t = 0; t < L; ++t) bc[t] = c[t];
-      }
-    }
-  }
-  // the winning group: lowest (E, entry) over the four groups' bests
-  int gw = -1, code = 0;
-  float ew = 0.f;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int kg = __builtin_amdgcn_readlane(bk, 16 * g);
-    const float eg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, best), 16 * g));
-    if (kg >= 0 && (gw < 0 || eg < ew || (eg == ew && kg < code))) {
-      gw = g;
-      ew = eg;
-      code = kg;
-    }
-  }
-  if (gw < 0) {  // no finite distance: code 0, as the strict-< scan from +inf leaves it
-    gw = 0;
-    if (grp == 0) {
-      const float* cr = cb + (int64_t)m * K * D + j * L;
-#pragma unroll
-      for (int t = 0; t < L; ++t) bc[t] = cr[t];
-    }
-  }
-  if (grp == gw) {
-    float a2 = 0.f;
-#pragma unroll
-    for (int t = 0; t < L; t += 4) {
-      float4 r4;
-      r4.x = rc[t] - bc[t];
-      r4.y = rc[t + 1] - bc[t + 1];
-      r4.z = rc[t + 2] - bc[t + 2];
-      r4.w = rc[t + 3] - bc[t + 3];
-      *reinterpret_cast<float4*>(&s.r[v][j * L + t]) = r4;
-      *reinterpret_cast<uint2*>(&s.rb[v][j * L + t]) = bf16x4_bits(r4);
-      a2 = __builtin_fmaf(r4.x, r4.x, a2);
-      a2 = __builtin_fmaf(r4.y, r4.y, a2);
-      a2 = __builtin_fmaf(r4.z, r4.z, a2);
-      a2 = __builtin_fmaf(r4.w, r4.w, a2);
-    }
-    a2 = row_fold16(a2);
-    if (j == 0) {
-      s.rn[v] = a2;
-      if (m < kCodeStage) s.code[v][m] = (uint8_t)code;
-      else if (row0 + v < N && rm.live(row0 + v)) rm.crow(row0 + v)[m] = (uint8_t)code;
-    }
-  }
-  lds_barrier();
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void encode_mfma4_kernel(
-    RowMap rm, int N, const float* __restrict__ cb, int M, int K,
-    const uint4* __restrict__ frag4, const float* __restrict__ cn,
-    const float* __restrict__ scn, float* __restrict__ rnorm) {
-  constexpr int L = D / 16;
-  __shared__ __attribute__((aligned(16))) Enc4Shared<D> s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row0 = blockIdx.x * kR4;
-  const int NQ = (K + 63) / 64;
-  const int qc = wave < NQ ? wave : NQ - 1;
-  if (rm.ranges) {  // a workgroup with no live row leaves at once (same test in every thread)
-    bool any = false;
-    for (int r = 0; r < kR4; ++r) any = any || (row0 + r < N && rm.live(row0 + r));
-    if (!any) return;
-  }
-  const int k = wave * 64 + lane;
-  const bool own = k < K;
-  const int kc = own ? k : K - 1;  // dead lanes load entry K - 1 (in bounds, ignored)
-  // Stage 0's operands are requested first, so that they arrive with the
-  // rows; stage m + 1's before stage m runs (unconditionally, the last stage
-  // re-requesting itself, so that the compiler's wait counts stay exact).
-  Enc4Stage<D> st0, st1;
-  enc4_load_stage<D>(st0, frag4, cn, scn, 0, NQ, K, qc, kc, lane);
-  for (int i = tid; i < kR4 * D; i += 256) {
-    const int r = i / D, d = i - r * D;
-    const float x = (row0 + r < N && rm.live(row0 + r)) ? rm.xval(row0 + r, d) : 0.f;
-    s.r[r][d] = x;
-    s.rb[r][d] = __builtin_bit_cast(uint16_t, (__bf16)x);
-  }
-  lds_barrier();
-  if (lane < 16) {  // wave v: dot16 norm of row v
-    const float* rr = s.r[wave] + lane * L;
-    float a2 = 0.f;
-#pragma unroll
-    for (int t = 0; t < L; ++t) a2 = __builtin_fmaf(rr[t], rr[t], a2);
-    a2 = row_fold16(a2);
-    if (lane == 0) s.rn[wave] = a2;
-  }
-  lds_barrier();
-
-  for (int m = 0; m < M; m += 2) {
-    enc4_load_stage<D>(st1, frag4, cn, scn, min(m + 1, M - 1), NQ, K, qc, kc, lane);
-    enc4_stage<D>(s, st0, cb, cn, m, K, row0, N, rm, own, k, wave, lane);
-    if (m + 1 >= M) break;
-    enc4_load_stage<D>(st0, frag4, cn, scn, min(m + 2, M - 1), NQ, K, qc, kc, lane);
-    enc4_stage<D>(s, st1, cb, cn, m + 1, K, row0, N, rm, own, k, wave, lane);
-  }
-  const int mc = M < kCodeStage ? M : kCodeStage;
-  for (int i = tid; i < kR4 * mc; i += 256) {
-    const int r = i / mc, mm = i - r * mc;
-    if (row0 + r < N && rm.live(row0 + r)) rm.crow(row0 + r)[mm] = s.code[r][mm];
-  }
-  if (tid < kR4 && rnorm && row0 + tid < N && rm.live(row0 + tid))
-    rnorm[row0 + tid] = sqrtf(s.rn[tid]);
-}
-
 // ------------------------------------------ exact distances (flushes)
-// A decode flush (8 KV heads x 64 tokens = 512 rows) has few rows per CU, and
-// the bf16-MFMA kernels above pay a chain of dependent latencies per stage:
-// coarse pass, survivor ballots, an L2 round trip for each survivor's fp32
-// row, the exact recheck, the residual update.  Here every stage computes
-// the contract's distance exactly for all K entries, with no coarse pass and
-// no survivors: thread k of the 256 owns entry k and holds that entry's fp32
-// row in registers (D values), loaded from the [M][D/4][K] float4 layout of
-// the prep (each wave instruction reads one contiguous kilobyte).  A stage:
+// Small flushes at D = 64.  Every stage computes the contract's distance exactly
+// for all K entries, with no coarse pass and no survivors: thread k of the 256
+// owns entry k and holds that entry's fp32 row in registers (D values), loaded
+// from the [M][D/4][K] float4 layout of the prep (each wave instruction reads
+// one contiguous kilobyte).  A stage:
 //   A. every thread runs the contract's dot16 (16 fmaf chains of D/16 and
 //      the fold) of its entry against each of the R residuals, read from LDS
 //      as broadcasts; each block of its row is reloaded with the next
 //      stage's as soon as its products are done, so that the codebook
 //      stream (every workgroup reads all of it) runs under the arithmetic;
 //      each wave then takes its minimum of (orderable distance, entry) with
-//      DPP and a ballot.  At C3 (two rows) the products' residual reads and
-//      the stream each take about 0.9 us of a stage's 2 us;
+//      DPP and a ballot;
 //   B. (after a barrier) wave v picks row v's winner among the four wave
 //      minima (lowest distance, then lowest entry; NaN and +inf never win;
 //      none finite: entry 0), reads that entry's row from the fp32
@@ -1265,10 +956,10 @@ extern "C" int lap_encode_prepare(const float* codebooks, int M, int K, int D, v
   hipLaunchKernelGGL(encode_prep_transpose, dim3((K + 31) / 32, (D + 31) / 32, M), dim3(256), 0,
                      st, codebooks, M, K, D, p.ct);
   LAP_LAUNCH_CHECK("encode_prep_transpose");
-  hipLaunchKernelGGL(encode_prep_norms, dim3((M * K + 255) / 256), dim3(256), 0, st, codebooks,
+  hipLaunchKernelGGL(encode_prep_norms, dim3((M * K + 15) / 16), dim3(256), 0, st, codebooks,
                      M, K, D, p.cn, p.scn);
   LAP_LAUNCH_CHECK("encode_prep_norms");
-  {
+  if (D == 64) {
     const int64_t n = (int64_t)M * (D / 4) * K;
     hipLaunchKernelGGL(encode_prep_c4, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
                        dim3(256), 0, st, codebooks, M, K, D, p.c4);
@@ -1276,22 +967,18 @@ extern "C" int lap_encode_prepare(const float* codebooks, int M, int K, int D, v
   }
   if (wide_serves(K, D)) {
     if (D == 64)
-      hipLaunchKernelGGL(encode_prep_wide<64>, dim3(M), dim3(256), 0, st, codebooks, M, K, p.cn,
+      hipLaunchKernelGGL(encode_prep_wide<64>, dim3(M), dim3(1024), 0, st, codebooks, M, K, p.cn,
                          p.wide, p.wstage);
     else
-      hipLaunchKernelGGL(encode_prep_wide<128>, dim3(M), dim3(256), 0, st, codebooks, M, K, p.cn,
+      hipLaunchKernelGGL(encode_prep_wide<128>, dim3(M), dim3(1024), 0, st, codebooks, M, K, p.cn,
                          p.wide, p.wstage);
     LAP_LAUNCH_CHECK("encode_prep_wide");
   }
-  if (K % 16 == 0) {
+  if (K % 16 == 0 && D == 256) {
     const int64_t n = (int64_t)M * (K / 16) * (D / 16) * 64;
     hipLaunchKernelGGL(encode_prep_frag, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                        codebooks, M, K, D, p.frag);
     LAP_LAUNCH_CHECK("encode_prep_frag");
-    const int64_t n4 = (int64_t)M * ((K + 63) / 64) * (D / 8) * 64;
-    hipLaunchKernelGGL(encode_prep_frag4, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st,
-                       codebooks, M, K, D, p.frag4);
-    LAP_LAUNCH_CHECK("encode_prep_frag4");
   }
   return LAP_OK;
 }
@@ -1301,53 +988,40 @@ static int encode_cus() {
   return device_info(&di) == LAP_OK ? di.cu_count : 256;
 }
 
-// Prompt-sized launches: the wide kernel (encode_wide.h).  It needs a wave per
-// 32 rows to fill the chip; below 32768 rows (half of the CUs with one
-// workgroup of 256 rows) the 16-row workgroups below keep more of them busy.
+// D = 64 and 128 (encode_wide.h).  More than 128 rows per CU: the wide kernel,
+// a wave per 32 rows; up to there the split kernel, whose stage is shorter but
+// which reads the stage's table for every 32 rows instead of 256 (D = 128, us:
+// 16384 rows 93 split, 32768 rows 179 split and 190-210 wide, 65536 rows 355
+// split and 230 wide; the 16- and 4-row bf16 kernels that they replaced took 90
+// for 2048 rows, 327 for 16384).
 // LAPRUNE_ENCODE_TILE=0|1 forces the choice (read at every call).
 static bool encode_use_wide(int N) {
   const char* e = getenv("LAPRUNE_ENCODE_TILE");
   if (e && (e[0] == '0' || e[0] == '1') && e[1] == 0) return e[0] == '1';
-  return (int64_t)N >= 128 * (int64_t)encode_cus();
+  return (int64_t)N > 128 * (int64_t)encode_cus();
 }
 
-// Small encodes (decode flushes) take the 4-row kernel while its workgroups
-// fit twice over on the chip; larger ones the 16-row kernel.
-// LAPRUNE_ENCODE_ROWS=4|16 forces the choice (D = 64 or 128); read at every
-// call, so that one process can run both.
-static bool encode_use_rows4(int N, int D) {
-  if (!(D == 64 || D == 128)) return false;
+// Rows per workgroup of the split kernel: 16 while that gives every CU at most
+// one workgroup (D = 128: 512 rows 55 us against 58 with 32, 4096 rows 60.5
+// against 63).  LAPRUNE_ENCODE_ROWS=16|32 forces it (read at every call).
+static int encode_split_rows(int N) {
   const char* e = getenv("LAPRUNE_ENCODE_ROWS");
   const int forced = e ? atoi(e) : 0;
-  if (forced == 4 || forced == 16) return forced == 4;
-  DevInfo di;
-  const int cus = device_info(&di) == LAP_OK ? di.cu_count : 256;
-  return (int64_t)(N + kR4 - 1) / kR4 <= 2 * (int64_t)cus;
+  if (forced == 16 || forced == 32) return forced;
+  return (int64_t)N <= 16 * (int64_t)encode_cus() ? 16 : 32;
 }
 
-// Flushes take the exact kernel while its workgroups fit once on the chip:
-// one row per workgroup up to one workgroup per CU, two rows up to twice
-// that (a 512-row C3 flush: 256 workgroups).  A workgroup streams the whole
-// codebook whatever its row count, so two workgroups on one CU take about
-// twice as long, and larger flushes go to the 4-row MFMA kernel.
-// LAPRUNE_ENCODE_EXACT=0|1 forces the choice and LAPRUNE_ENCODE_EXACT_ROWS=1|2
-// the rows per workgroup; LAPRUNE_ENCODE_ROWS=4|16 (a forced MFMA kernel)
-// turns it off.  All are read at every call, so that one process can compare
-// them.
-static int encode_exact_rows(int N) {
-  const char* e = getenv("LAPRUNE_ENCODE_EXACT_ROWS");
-  const int r = e ? atoi(e) : 0;
-  if (r == 1 || r == 2) return r;
-  return N <= encode_cus() ? 1 : 2;
-}
+// At D = 64, up to one row per CU, the exact kernel (33.5 us for up to 256 rows
+// against 39.6 split; at D = 128 its stream of the fp32 codebook takes longer
+// than the split kernel's stage: 57-60 us against 50-52).
+// LAPRUNE_ENCODE_EXACT=0|1 forces it where it is built (D = 64);
+// LAPRUNE_ENCODE_ROWS turns it off (both read at every call).
 static bool encode_use_exact(int N, int D, int K) {
-  if (!(D == 64 || D == 128) || K > 256) return false;
+  if (D != 64 || K > 256) return false;
   const char* e = getenv("LAPRUNE_ENCODE_EXACT");
   if (e && (e[0] == '0' || e[0] == '1') && e[1] == 0) return e[0] == '1';
-  const char* rows = getenv("LAPRUNE_ENCODE_ROWS");
-  if (rows && (atoi(rows) == 4 || atoi(rows) == 16)) return false;
-  if (!encode_impl_mfma()) return false;
-  return (int64_t)(N + 1) / 2 <= encode_cus();
+  if (getenv("LAPRUNE_ENCODE_ROWS") || !encode_impl_mfma()) return false;
+  return N <= encode_cus();
 }
 
 // Rows whose chunks the wide kernel may read as vectors.
@@ -1378,6 +1052,23 @@ static int launch_wide(const RowMap& rm, int N, int D, const float* cb, int M, i
   return launch_wide_as<128, 8>(rm, N, cb, M, K, p, rnorm, st);
 }
 
+static int launch_split(const RowMap& rm, int N, int D, const float* cb, int M, int K,
+                        const Prep& p, float* rnorm, hipStream_t st) {
+  const int rows = encode_split_rows(N);
+  const dim3 grid((N + rows - 1) / rows);
+#define LAP_ENCS(D_, R_)                                                                      \
+  hipLaunchKernelGGL((encode_split_kernel<D_, R_>), grid, dim3(512), 0, st, rm, N, cb, M, K, \
+                     p.wide, p.wstage, p.cn, rnorm)
+  if (D == 64) {
+    if (rows == 16) LAP_ENCS(64, 16); else LAP_ENCS(64, 32);
+  } else {
+    if (rows == 16) LAP_ENCS(128, 16); else LAP_ENCS(128, 32);
+  }
+#undef LAP_ENCS
+  LAP_LAUNCH_CHECK("encode_split_kernel");
+  return LAP_OK;
+}
+
 // Shared checks and launch of both encode entry points.
 static int run_encode(const RowMap& rm, int N, int D, const float* codebooks, int M, int K,
                       const void* prep, size_t prep_bytes, float* resid_norm,
@@ -1398,44 +1089,19 @@ static int run_encode(const RowMap& rm, int N, int D, const float* codebooks, in
   if (N == 0) return LAP_OK;
   hipStream_t st = as_stream(stream);
   if (encode_use_exact(N, D, K)) {
-    const int R = encode_exact_rows(N);
-    dim3 g((N + R - 1) / R);
-#define LAP_ENCX(D_, R_)                                                                 \
-  hipLaunchKernelGGL((encode_exact_kernel<D_, R_>), g, dim3(256), 0, st, rm, N, codebooks, \
-                     p.c4, p.cn, M, K, resid_norm)
-    if (D == 64) {
-      if (R == 1) LAP_ENCX(64, 1); else LAP_ENCX(64, 2);
-    } else {
-      if (R == 1) LAP_ENCX(128, 1); else LAP_ENCX(128, 2);
-    }
-#undef LAP_ENCX
+    hipLaunchKernelGGL((encode_exact_kernel<64, 1>), dim3(N), dim3(256), 0, st, rm, N, codebooks,
+                       p.c4, p.cn, M, K, resid_norm);
     LAP_LAUNCH_CHECK("encode_exact_kernel");
     return LAP_OK;
   }
-  if (wide_serves(K, D) && encode_impl_mfma() && encode_use_wide(N))
-    return launch_wide(rm, N, D, codebooks, M, K, p, resid_norm, st);
-  if (K % 16 == 0 && encode_impl_mfma() && encode_use_rows4(N, D)) {
-    dim3 g4((N + kR4 - 1) / kR4);
-    const uint4* fr = reinterpret_cast<const uint4*>(p.frag4);
-    if (D == 64)
-      hipLaunchKernelGGL(encode_mfma4_kernel<64>, g4, dim3(256), 0, st, rm, N, codebooks, M, K,
-                         fr, p.cn, p.scn, resid_norm);
-    else
-      hipLaunchKernelGGL(encode_mfma4_kernel<128>, g4, dim3(256), 0, st, rm, N, codebooks, M, K,
-                         fr, p.cn, p.scn, resid_norm);
-    LAP_LAUNCH_CHECK("encode_mfma4_kernel");
-    return LAP_OK;
-  }
+  if (wide_serves(K, D) && encode_impl_mfma())
+    return encode_use_wide(N) ? launch_wide(rm, N, D, codebooks, M, K, p, resid_norm, st)
+                              : launch_split(rm, N, D, codebooks, M, K, p, resid_norm, st);
   if (K % 16 == 0 && encode_impl_mfma()) {
     dim3 g16((N + 15) / 16);
     const uint2* fr = reinterpret_cast<const uint2*>(p.frag);
-#define LAP_ENCM(D_)                                                                         \
-  hipLaunchKernelGGL(encode_mfma_kernel<D_>, g16, dim3(EncCfg<D_>::THREADS), 0, st, rm, N,   \
-                     codebooks, M, K, fr, p.cn, p.scn, resid_norm)
-    if (D == 64) LAP_ENCM(64);
-    else if (D == 128) LAP_ENCM(128);
-    else LAP_ENCM(256);
-#undef LAP_ENCM
+    hipLaunchKernelGGL(encode_mfma_kernel<256>, g16, dim3(EncCfg<256>::THREADS), 0, st, rm, N,
+                       codebooks, M, K, fr, p.cn, p.scn, resid_norm);
     LAP_LAUNCH_CHECK("encode_mfma_kernel");
     return LAP_OK;
   }

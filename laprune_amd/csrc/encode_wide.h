@@ -75,50 +75,48 @@ __device__ __forceinline__ float wide_f16_flushed(float x) {
 // fragments.  Entries past K repeat entry K - 1 (they can then neither raise
 // the maximum nor be picked).
 template <int D>
-__global__ __launch_bounds__(256) void encode_prep_wide(const float* __restrict__ cb, int M,
-                                                        int K, const float* __restrict__ cn,
-                                                        uint4* __restrict__ wide,
-                                                        WideStage* __restrict__ stage) {
-  constexpr int KS = D / 16;
-  __shared__ float s_max[256], s_err[256];
+__global__ __launch_bounds__(1024) void encode_prep_wide(const float* __restrict__ cb, int M,
+                                                         int K, const float* __restrict__ cn,
+                                                         uint4* __restrict__ wide,
+                                                         WideStage* __restrict__ stage) {
+  constexpr int KS = D / 16, L = D / 16;
+  __shared__ float s_red[16];
   const int m = blockIdx.x, tid = threadIdx.x;
   const float* cbm = cb + (int64_t)m * K * D;
   const float* cnm = cn + (int64_t)m * K;
-  auto block_max = [&](float* s, float v) {
-    s[tid] = v;
+  auto block_max = [&](float v) {
+    for (int w = 32; w >= 1; w >>= 1) v = fmaxf(v, __shfl_xor(v, w, 64));
+    if ((tid & 63) == 0) s_red[tid >> 6] = v;
     __syncthreads();
-    for (int w = 128; w >= 1; w >>= 1) {
-      if (tid < w) s[tid] = fmaxf(s[tid], s[tid + w]);
-      __syncthreads();
-    }
-    const float r = s[0];
+    float r = s_red[0];
+    for (int i = 1; i < 16; ++i) r = fmaxf(r, s_red[i]);
     __syncthreads();
     return r;
   };
-  float mx = 0.f;
-  bool bad = false;
-  for (int k = tid; k < K; k += 256) {
-    const float v = cnm[k];
-    bad = bad || !(v < 0x1p24f);  // NaN, inf or a norm of 2^12 and above
-    mx = fmaxf(mx, v);
-  }
-  bad = __syncthreads_or(bad);
-  const float cmax = block_max(s_max, mx);
+  const float v = tid < K ? cnm[tid] : 0.f;
+  const bool bad = __syncthreads_or(!(v < 0x1p24f));  // NaN, inf or a norm of 2^12 and above
+  const float cmax = block_max(v);
   int b = cmax > 0.f && !bad ? 9 - ilogbf(sqrtf(cmax)) : 0;
   b = b < -20 ? -20 : b > 60 ? 60 : b;
   const float sc = ldexpf(1.f, b);
-  // the largest rounding-error norm of the stage's fp16 entries
+  // the largest rounding-error norm of the stage's fp16 entries, four threads
+  // per entry
   float err = 0.f;
-  for (int k = tid; k < K; k += 256) {
-    float e = 0.f;
-    for (int d = 0; d < D; ++d) {
-      const float x = cbm[(int64_t)k * D + d] * sc;
-      const float dx = x - wide_f16_flushed(x);
-      e = __builtin_fmaf(dx, dx, e);
+  if (tid / 4 < K) {
+    const float* row = cbm + (int64_t)(tid / 4) * D + (tid & 3) * 4;
+    for (int d = 0; d < D; d += 16) {
+      const float4 x = *reinterpret_cast<const float4*>(row + d);
+      const float xs[4] = {x.x * sc, x.y * sc, x.z * sc, x.w * sc};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float dx = xs[e] - wide_f16_flushed(xs[e]);
+        err = __builtin_fmaf(dx, dx, err);
+      }
     }
-    err = fmaxf(err, e);
   }
-  const float d_ = sqrtf(block_max(s_err, err)) * 1.001f;
+  err += __shfl_xor(err, 1, 64);
+  err += __shfl_xor(err, 2, 64);
+  const float d_ = sqrtf(block_max(err)) * 1.001f;
   if (tid == 0) {
     const float c = sqrtf(cmax) * sc * 1.001f, h = 0.5f * cmax * sc * 1.001f;
     WideStage w;
@@ -131,26 +129,32 @@ __global__ __launch_bounds__(256) void encode_prep_wide(const float* __restrict_
   }
   const int NT = wide_tiles(K), nf = NT * KS * 64;
   uint4* out = wide + (int64_t)m * wide_stage_uint4(K, D);
-  for (int i = tid; i < nf; i += 256) {
+  for (int i = tid; i < nf; i += 1024) {
     const int l = i & 63, ks = (i >> 6) % KS, tile = (i >> 6) / KS;
     const int k = min(32 * tile + (l & 31), K - 1);
-    wh8_t v;
+    const float* row = cbm + (int64_t)k * D;
+    wh8_t x;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = __builtin_bit_cast(_Float16, f2h(cbm[(int64_t)k * D + wide_dim<D>(ks, e, l >> 5)] * sc));
-    out[i] = __builtin_bit_cast(uint4, v);
+    for (int e = 0; e < 8; e += 4) {  // four slots in a row are four dimensions in a row
+      static_assert(L % 4 == 0, "chains of whole float4 blocks");
+      const float4 y = *reinterpret_cast<const float4*>(row + wide_dim<D>(ks, e, l >> 5));
+      x[e] = __builtin_bit_cast(_Float16, f2h(y.x * sc));
+      x[e + 1] = __builtin_bit_cast(_Float16, f2h(y.y * sc));
+      x[e + 2] = __builtin_bit_cast(_Float16, f2h(y.z * sc));
+      x[e + 3] = __builtin_bit_cast(_Float16, f2h(y.w * sc));
+    }
+    out[i] = __builtin_bit_cast(uint4, x);
   }
   uint2* hp = reinterpret_cast<uint2*>(out + nf);
-  for (int i = tid; i < (int)(wide_stage_uint4(K, D) - nf) * 2; i += 256) {
-    const int k = min(i, K - 1);
-    float x = cnm[k] * (0.5f * sc) * 0x1p-6f;
-    wh4_t v = {};
+  for (int i = tid; i < (int)(wide_stage_uint4(K, D) - nf) * 2; i += 1024) {
+    float x = cnm[min(i, K - 1)] * (0.5f * sc) * 0x1p-6f;
+    wh4_t y = {};
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
-      v[e] = __builtin_bit_cast(_Float16, f2h(x));
-      x = x - (float)v[e];
+      y[e] = __builtin_bit_cast(_Float16, f2h(x));
+      x = x - (float)y[e];
     }
-    hp[i] = __builtin_bit_cast(uint2, v);
+    hp[i] = __builtin_bit_cast(uint2, y);
   }
 }
 
@@ -529,6 +533,298 @@ __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
 #pragma unroll
   for (int u = 0; u < 2; ++u)
     if (q == 0 && live[u] && rnorm) rnorm[row0 + 16 * u] = sqrtf(rn[u]);
+}
+
+// ------------------------------------------ fewer rows than the chip has waves
+// The same search and update for up to about two workgroups per CU, where the
+// chain of a stage's dependent steps sets the time: R = 32 or 16 rows per
+// workgroup of eight waves.  Wave w searches tile w for all R rows (its
+// fragments come straight from L2 into registers, the next stage's requested
+// as soon as this one's products are issued) and updates R / 8 rows, sixteen
+// lanes per row, lane j the dot16 chain j; a maximum and a survivor mask per
+// (row, tile) and the fp16 residual change hands through LDS, two barriers per
+// stage.  R = 16 (16x16x32 products, half the work between the barriers) while
+// every CU gets at most one workgroup of 16 rows.
+constexpr int kSplitCodes = 32;  // codes of the first stages, stored after the last
+
+template <int D, int R>
+struct SplitShared {
+  uint4 b[R * (D / 8)];  // fp16 residual, 16-byte units of a row permuted by the row
+  uint2 m[R][8];         // per row and tile: maximum, entries within 2 eps of it
+  float eps2[R];
+  uint8_t code[R][kSplitCodes];
+};
+
+typedef float wf4_t __attribute__((ext_vector_type(4)));
+
+// Maximum and union over lanes l, l ^ 16, l ^ 32, l ^ 48, in all of them.
+__device__ __forceinline__ float quarter_max(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, half_max(x));
+  const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t a = p[0], b = p[1];  // (a bit cast of the element itself reads element 0)
+  return __builtin_elementwise_maximum(__builtin_bit_cast(float, a),
+                                       __builtin_bit_cast(float, b));
+}
+__device__ __forceinline__ uint32_t quarter_or(uint32_t x) {
+  const HalfPair h = halves(x);
+  const auto p = __builtin_amdgcn_permlane16_swap(h.lo | h.hi, h.lo | h.hi, false, false);
+  return p[0] | p[1];
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false);
+}
+
+template <int D, int R>
+__global__ __launch_bounds__(512, 4) void encode_split_kernel(
+    RowMap rm, int N, const float* __restrict__ cb, int M, int K,
+    const uint4* __restrict__ wide, const WideStage* __restrict__ stage,
+    const float* __restrict__ cn, float* __restrict__ rnorm) {
+  constexpr int KS = D / 16, L = D / 16, U = D / 8;  // units per row
+  constexpr uint32_t kNone = 0x7fffu;
+  static_assert(R == 16 || R == 32, "rows per workgroup");
+  __shared__ __attribute__((aligned(16))) SplitShared<D, R> s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // search: row, and the half (R = 32) or quarter of the wave
+  const int n = lane & (R - 1), h = lane / R;
+  const int j = lane & 15;  // update: chain
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // update: row (R = 16: the upper half of the wave repeats the lower)
+  const int lrow = R / 8 * wave + ((lane >> 4) & (R / 8 - 1)), row = blockIdx.x * R + lrow;
+  const int NT = wide_tiles(K);
+  const int64_t n16 = wide_stage_uint4(K, D);
+  const bool live = row < N && rm.live(row);
+  // a workgroup with no live row leaves at once
+  if (rm.ranges && !__syncthreads_or(live)) return;
+
+  // Waves past the last tile load it again and offer nothing.
+  const int tile = min(wave, NT - 1);
+  // bits of a tile's mask that stand for entries (entry e at bit 31 - e)
+  auto entries = [&](int t) -> uint32_t {
+    const int c = K - 32 * t;
+    return c >= 32 ? ~0u : c > 0 ? ~0u << (32 - c) : 0u;
+  };
+  const uint32_t mine = wave < NT ? entries(wave) : 0u, theirs = entries(j & 7);
+  // stage m's fragments of the tile: a uniform base each, and the lane.
+  // Slot i: 32 rows, k-step i; 16 rows, k-steps 2 (i / 2) and 2 (i / 2) + 1 of
+  // the tile's 16 entries i % 2 (operand A's quarter q is k-step q / 2, half
+  // q % 2 of the pair).
+  uint4 f[KS];
+  uint2 hp[R == 32 ? 1 : 2];
+  auto fragment = [&](int m, int i) {
+    const uint4* base = wide + m * n16 + tile * KS * 64;
+    return R == 32 ? base[i * 64 + lane]
+                   : base[(i & ~1) * 64 + (i & 1) * 16 + (h >> 1) * 64 + (h & 1) * 32 + n];
+  };
+  auto part = [&](int m, int x) {
+    return reinterpret_cast<const uint2*>(wide + m * n16 + NT * KS * 64)[tile * 32 + x * 16 + n];
+  };
+#pragma unroll
+  for (int x = 0; x < (R == 32 ? 1 : 2); ++x) hp[x] = part(0, x);
+#pragma unroll
+  for (int i = 0; i < KS; ++i) f[i] = fragment(0, i);
+
+  float r[L];
+#pragma unroll
+  for (int t = 0; t < L; ++t) r[t] = live ? rm.xval(row, j * L + t) : 0.f;
+  float rn = 0.f, eps2 = 0.f;
+  // new norm, 2 eps and fp16 residual of the row
+  auto publish = [&](const WideStage& ws) {
+    float a = 0.f;
+#pragma unroll
+    for (int t = 0; t < L; ++t) a = __builtin_fmaf(r[t], r[t], a);
+    rn = row_fold16(a);
+    eps2 = __builtin_fmaf(__builtin_amdgcn_sqrtf(rn), ws.e1, __builtin_fmaf(rn, ws.e2, ws.e0));
+    if (j == 0) s.eps2[lrow] = eps2;
+    if constexpr (L == 8) {  // chain j is unit j
+      wh8_t x;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) x[t] = (_Float16)r[t];
+      s.b[lrow * U + (j ^ (lrow & 15))] = __builtin_bit_cast(uint4, x);
+    } else {  // L = 4: chains 8v + q and 8v + 4 + q are the halves of unit 4v + q
+      wh4_t x;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = (_Float16)r[t];
+      const int u = 4 * (j >> 3) + (j & 3);
+      reinterpret_cast<uint2*>(s.b)[(lrow * U + (u ^ (lrow & 7))) * 2 + ((j >> 2) & 1)] =
+          __builtin_bit_cast(uint2, x);
+    }
+  };
+  publish(stage[0]);
+  wh4_t baug = {};
+  if (h == 0) baug[0] = baug[1] = baug[2] = (_Float16)-64.f;
+  lds_barrier();
+
+  for (int m = 0; m < M; ++m) {
+    const int mn = min(m + 1, M - 1);
+    // ---- search: rows n, tile `tile`.  Each fragment's successor is requested
+    // as soon as its product is issued: the eight waves' requests take the
+    // vector memory unit about 1150 cycles, and issued in one block they held
+    // up the sifting (and, issued later, the candidates' rows).
+    const float re = s.eps2[n];
+    const WideStage ws = stage[mn];
+    float x;
+    uint32_t w;  // the tile's entries within 2 eps of its maximum, entry e at bit 31 - e
+    const uint4* br = s.b + n * U;
+    if constexpr (R == 32) {
+      wf16_t a = {};
+      wh8_t bf[KS];
+#pragma unroll
+      for (int i = 0; i < KS; ++i)
+        bf[i] = __builtin_bit_cast(wh8_t, br[(2 * i + h) ^ (n & (U - 1))]);
+      a = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(wh4_t, hp[0]), baug, a, 0, 0, 0);
+      hp[0] = part(mn, 0);
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        a = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(wh8_t, f[i]), bf[i], a, 0, 0,
+                                                   0);
+        f[i] = fragment(mn, i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float y = __builtin_elementwise_maximum(a[2], a[3]);
+      x = __builtin_elementwise_maximum(a[0], a[1]);
+#pragma unroll
+      for (int i = 4; i < 16; i += 4) {
+        x = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, a[i]), a[i + 1]);
+        y = __builtin_elementwise_maximum(__builtin_elementwise_maximum(y, a[i + 2]), a[i + 3]);
+      }
+      x = half_max(__builtin_elementwise_maximum(x, y));
+      const float thr = x - re;
+      uint32_t w0 = 0, w1 = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        w0 = __builtin_amdgcn_alignbit(w0, __builtin_bit_cast(uint32_t, a[i] - thr), 31);
+        w1 = __builtin_amdgcn_alignbit(w1, __builtin_bit_cast(uint32_t, a[8 + i] - thr), 31);
+      }
+      w = ~((w0 << 8) | w1) & 0xffffu;  // register i at bit 15 - i
+      // registers 4g .. 4g + 3 of half h are entries 8g + 4h ..
+      w = (w | (w << 8)) & 0x00ff00ffu;
+      w = (w | (w << 4)) & 0x0f0f0f0fu;
+      const HalfPair wp = halves(w);
+      w = (wp.lo << 4) | wp.hi;
+    } else {
+      wf4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      wh8_t bf[KS / 2];
+#pragma unroll
+      for (int i = 0; i < KS / 2; ++i)
+        bf[i] = __builtin_bit_cast(wh8_t, br[(4 * i + h) ^ (n & (U - 1))]);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        a[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(wh4_t, hp[e]), baug, a[e],
+                                                     0, 0, 0);
+        hp[e] = part(mn, e);
+      }
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        a[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(wh8_t, f[i]),
+                                                          bf[i / 2], a[i & 1], 0, 0, 0);
+        f[i] = fragment(mn, i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      x = __builtin_elementwise_maximum(a[0][0], a[0][1]);
+      float y = __builtin_elementwise_maximum(a[1][0], a[1][1]);
+      x = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, a[0][2]), a[0][3]);
+      y = __builtin_elementwise_maximum(__builtin_elementwise_maximum(y, a[1][2]), a[1][3]);
+      x = quarter_max(__builtin_elementwise_maximum(x, y));
+      const float thr = x - re;
+      uint32_t w0 = 0, w1 = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        w0 = __builtin_amdgcn_alignbit(w0, __builtin_bit_cast(uint32_t, a[0][i] - thr), 31);
+        w1 = __builtin_amdgcn_alignbit(w1, __builtin_bit_cast(uint32_t, a[1][i] - thr), 31);
+      }
+      // register i of quarter h is entry 4h + i of the 16
+      w = quarter_or((((~w0 & 15u) << 16) | (~w1 & 15u)) << (12 - 4 * h));
+    }
+    if (h == 0)
+      s.m[n][wave] = make_uint2(mine ? __builtin_bit_cast(uint32_t, x) : 0xff800000u, w & mine);
+    lds_barrier();
+
+    // ---- update: row lrow, lanes j; lanes 8 .. 15 repeat tiles 0 .. 7
+    const float* cbm = cb + (int64_t)m * K * D + j * L;
+    const float* cnm = cn + (int64_t)m * K;
+    const uint2 mw = s.m[lrow][j & 7];
+    const float mx = __builtin_bit_cast(float, mw.x);
+    float top = __builtin_elementwise_maximum(mx, dpp_f<0x124>(mx));
+    top = __builtin_elementwise_maximum(top, dpp_f<0x122>(top));
+    top = __builtin_elementwise_maximum(top, dpp_f<0x121>(top));
+    const bool all = !(eps2 < 0x1p60f) || !(rn < 0x1p30f);  // outside the fp16 range
+    uint32_t keep = all ? theirs : mx >= top - eps2 ? mw.y : 0u;
+    uint32_t cnt = (uint32_t)__builtin_popcount(keep);
+    cnt += dpp_u32<0x124>(cnt);
+    cnt += dpp_u32<0x122>(cnt);
+    cnt += dpp_u32<0x121>(cnt);
+    // lowest candidate of the row (kNone: none); drop: takes it out
+    auto lowest = [&](bool drop) -> uint32_t {
+      const uint32_t b = (uint32_t)__builtin_clz(keep | 1u);
+      const uint32_t own = keep ? 32u * (uint32_t)(j & 7) + b : kNone;
+      uint32_t c = min(own, dpp_u32<0x124>(own));
+      c = min(c, dpp_u32<0x122>(c));
+      c = min(c, dpp_u32<0x121>(c));
+      if (drop && own == c && c != kNone) keep &= ~(0x80000000u >> b);
+      return c;
+    };
+    auto fetch = [&](float (&c)[L], uint32_t k) {
+#pragma unroll
+      for (int t = 0; t < L; t += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(cbm + (int64_t)k * D + t);
+        c[t] = v.x;
+        c[t + 1] = v.y;
+        c[t + 2] = v.z;
+        c[t + 3] = v.w;
+      }
+    };
+    const uint32_t ca = lowest(false);
+    int code = ca == kNone ? 0 : (int)ca;
+    float c[L];
+    fetch(c, (uint32_t)code);
+    if (__ballot(cnt > 1)) {
+      // as in the wide kernel: the contract's distances decide between several
+      // candidates, the lowest entry on a tie; NaN and +inf never win.  Rows
+      // without a second candidate read entry 0.
+      const float cna = cnm[code];
+      if (((uint32_t)code >> 5) == (uint32_t)(j & 7)) keep &= ~(0x80000000u >> (code & 31));
+      uint32_t cd = lowest(true);
+      float d[L], cnd = cnm[cd == kNone ? 0 : cd];
+      fetch(d, cd == kNone ? 0 : cd);
+      auto distance = [&](const float (&v)[L], float cnk) {
+        float dot = 0.f;
+#pragma unroll
+        for (int t = 0; t < L; ++t) dot = __builtin_fmaf(r[t], v[t], dot);
+        return (rn + cnk) - 2.0f * row_fold16(dot);
+      };
+      float best = distance(c, cna);
+      bool have = !(best != best) && best != INFINITY;
+      for (;;) {
+        const float E = distance(d, cnd);
+        const bool win = cd != kNone && !(E != E) && E != INFINITY && (!have || E < best);
+        best = win ? E : best;
+        code = win ? (int)cd : code;
+        have = have || win;
+#pragma unroll
+        for (int t = 0; t < L; ++t) c[t] = win ? d[t] : c[t];
+        cd = lowest(true);
+        if (!__ballot(cd != kNone)) break;
+        cnd = cnm[cd == kNone ? 0 : cd];
+        fetch(d, cd == kNone ? 0 : cd);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < L; ++t) r[t] = r[t] - c[t];
+    publish(ws);
+    if (j == 0) {
+      if (m < kSplitCodes) s.code[lrow][m] = (uint8_t)code;
+      else if (live) rm.crow(row)[m] = (uint8_t)code;
+    }
+    lds_barrier();
+  }
+  const int mc = M < kSplitCodes ? M : kSplitCodes;
+  for (int i = tid; i < R * mc; i += 512) {
+    const int rr = i / mc, mm = i - rr * mc, gr = blockIdx.x * R + rr;
+    if (gr < N && rm.live(gr)) rm.crow(gr)[mm] = s.code[rr][mm];
+  }
+  if (j == 0 && live && rnorm) rnorm[row] = sqrtf(rn);
 }
 
 }  // namespace

@@ -1,8 +1,8 @@
-"""The prompt-sized encode (encode_wide_kernel, 256 rows per workgroup), forced
-at the sizes where it can go wrong: codes and residual norms equal the oracle's
-bit for bit.
+"""The encode's wide and split kernels (256 rows, and 16 or 32 rows per workgroup),
+forced at the sizes where they can go wrong: codes and residual norms equal the
+oracle's bit for bit.
 
-Its coarse fp16 search may only rule entries out, so every case whose
+The coarse fp16 search may only rule entries out, so every case whose
 magnitudes leave the fp16 range (rows past 2^15, non-finite rows, codebook
 norms that are zero, tiny, past 2^12 or not finite) has to fall back to the
 contract's distances and give the same codes.
@@ -22,10 +22,14 @@ def K(dev):
     return aq_kernels
 
 
-@pytest.fixture()
-def wide(monkeypatch):
-    monkeypatch.setenv("LAPRUNE_ENCODE_TILE", "1")
+@pytest.fixture(params=["wide", "split16", "split32"])
+def wide(request, monkeypatch):
+    """Forces the wide kernel, or the split kernel with 16 or 32 rows per
+    workgroup (the environment is read at every call)."""
+    monkeypatch.setenv("LAPRUNE_ENCODE_TILE", "1" if request.param == "wide" else "0")
     monkeypatch.setenv("LAPRUNE_ENCODE_EXACT", "0")
+    if request.param != "wide":
+        monkeypatch.setenv("LAPRUNE_ENCODE_ROWS", request.param[5:])
 
 
 def _check(K, orc, dev, x, cb, what):
