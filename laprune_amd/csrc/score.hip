@@ -264,6 +264,121 @@ __global__ __launch_bounds__(THREADS) void score_g4p_kernel(
   }
 }
 
+// Scorer for any group size G = 1 .. 8 over the reference's per-head tables
+// [R * G][32][256].  HB = 1 or 2 blocks of four heads: a KV row's tables sit in
+// LDS as HB interleaved [32][256][4] tables of 64 KiB, so each code row is read
+// once and every lookup serves four heads; lanes of heads past G repeat head
+// G - 1 (a group maximum does not see them, and they are not written).  One
+// head per workgroup with two-byte lookups, which it replaced where the code
+// rows are aligned, read each code row G times and left the keys to a pass of
+// their own (G = 8, 4 x 65537 tokens: 27.4 us, here 12.3; G = 7, two sequences of
+// 4 x 50001 tokens: 2 x 22 and 18.5 us, here 12.9).  The lookups bound it: 64 per
+// token at G > 4, about six cycles per 64 lanes each, and the 128 KiB table fill
+// of every workgroup (about 2.5 us).  Outputs as
+// score_g4p_kernel: fp16 scores per head, or selection keys (group maximum, or
+// each head's with PH) and the chunk's 256-bin histograms of their high byte.
+// A workgroup owns `tok` stages of THREADS consecutive tokens of one row and
+// requests a stage's code rows under the stage before.
+template <int HB, bool PH>
+__global__ __launch_bounds__(1024) void score_any_kernel(
+    const uint16_t* __restrict__ lut, const uint8_t* __restrict__ codes, int64_t cs_b,
+    int64_t cs_h, int64_t cs_t, int Hkv, int G, int R, int T, int tok, ScoreOut so, _Float16 one) {
+  constexpr int TH = 1024, HC = PH ? 2 : 8;
+  constexpr int kGroups = kM * kK / 8;  // 8-entry groups per head table
+  extern __shared__ __attribute__((aligned(16))) uint4 any_smem[];
+  uint4* s_lut = any_smem;  // [HB][kLutBytes / 16]
+  uint32_t* s_hist = reinterpret_cast<uint32_t*>(s_lut + HB * (kLutBytes / 16));
+  const int r = blockIdx.x % R, chunk = blockIdx.x / R, tid = threadIdx.x;
+  const int rows = PH ? G : 1;  // selection rows of this KV row
+  const int b = r / Hkv, hkv = r - b * Hkv;
+  RowCols rc{T, so.cand_start, so.cand_end};
+  if (so.plans) rc = row_cols(so, b, T);
+  const int t0 = chunk * tok * TH, t1 = min(rc.t_end, t0 + tok * TH);
+  uint32_t* hist = so.hist ? so.hist + ((int64_t)r * rows * (gridDim.x / R) + chunk) * 256 : nullptr;
+  const int64_t hist_row = (int64_t)(gridDim.x / R) * 256;
+  if (t0 >= t1) {  // a chunk past the row's columns (same test in every thread)
+    if (hist)
+      for (int i = tid; i < rows * 256; i += TH) hist[(i >> 8) * hist_row + (i & 255)] = 0;
+    return;
+  }
+  const uint16_t* tab = lut + (int64_t)r * G * (kM * kK);
+  u32x4 f[HB][4];
+#pragma unroll
+  for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      f[hb][g] = *reinterpret_cast<const u32x4*>(tab + (int64_t)min(4 * hb + g, G - 1) * (kM * kK) +
+                                                 (tid & (kGroups - 1)) * 8);
+  const uint8_t* crow = codes + (int64_t)b * cs_b + (int64_t)hkv * cs_h;
+  uint4 c0, c1;
+  auto request = [&](int j) {
+    // rows past the chunk end load its last row (in bounds) and are dropped
+    const uint8_t* p = crow + (int64_t)min(t0 + j * TH + tid, t1 - 1) * cs_t;
+    c0 = *reinterpret_cast<const uint4*>(p);
+    c1 = *reinterpret_cast<const uint4*>(p + 16);
+  };
+  static_assert(kGroups == TH, "one group of eight entries per thread");
+#pragma unroll
+  for (int hb = 0; hb < HB; ++hb)
+    interleave_heads(f[hb][0], f[hb][1], f[hb][2], f[hb][3],
+                     s_lut + hb * (kLutBytes / 16) + tid * 4);
+  request(0);
+  if (hist)
+    for (int i = tid; i < rows * HC * kHPitch; i += TH) s_hist[i] = 0;
+  lds_barrier();
+
+  const char* lds = reinterpret_cast<const char*>(s_lut);
+  const uint32_t copy = (uint32_t)(__lane_id() % HC) * kHPitch;
+  const int lo = max(rc.cs, 0), hi = min(rc.ce, t1);  // histogram window in this chunk
+  const bool kbf = so.key_mode == LAP_KEY_BF16;
+  for (int j = 0; j < tok && t0 + j * TH < t1; ++j) {
+    const uint4 w0 = c0, w1 = c1;
+    if (j + 1 < tok) request(j + 1);
+    float e[HB][4];
+#pragma unroll
+    for (int hb = 0; hb < HB; ++hb) {
+      e[hb][0] = e[hb][1] = e[hb][2] = e[hb][3] = 0.f;
+      score_token(lds + hb * kLutBytes, w0, w1, one, e[hb][0], e[hb][1], e[hb][2], e[hb][3]);
+    }
+    const int t = t0 + j * TH + tid;
+    if (t >= t1) continue;
+    const bool counted = hist && t >= lo && t < hi;
+    if (so.heads) {
+      uint16_t* hp = so.heads + (int64_t)r * G * T + t;
+#pragma unroll
+      for (int g = 0; g < 4 * HB; ++g)
+        if (g < G) hp[(int64_t)g * T] = f2h(e[g >> 2][g & 3]);
+    }
+    if (!so.keys) continue;
+    if constexpr (PH) {
+      uint16_t* kp = so.keys + (int64_t)r * G * T + t;
+#pragma unroll
+      for (int g = 0; g < 4 * HB; ++g)
+        if (g < G) {
+          const uint32_t key = key_of_score(e[g >> 2][g & 3], kbf);
+          kp[(int64_t)g * T] = (uint16_t)key;
+          if (counted) atomicAdd(&s_hist[g * HC * kHPitch + copy + (key >> 8)], 1u);
+        }
+    } else {
+      float mx = fmaxf(fmaxf(e[0][0], e[0][1]), fmaxf(e[0][2], e[0][3]));
+      if constexpr (HB == 2)
+        mx = fmaxf(mx, fmaxf(fmaxf(e[1][0], e[1][1]), fmaxf(e[1][2], e[1][3])));
+      const uint32_t key = key_of_score(mx, kbf);
+      so.keys[(int64_t)r * T + t] = (uint16_t)key;
+      if (counted) atomicAdd(&s_hist[copy + (key >> 8)], 1u);
+    }
+  }
+  if (hist) {
+    __syncthreads();
+    for (int i = tid; i < rows * 256; i += TH) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int c = 0; c < HC; ++c) v += s_hist[((i >> 8) * HC + c) * kHPitch + (i & 255)];
+      hist[(i >> 8) * hist_row + (i & 255)] = v;
+    }
+  }
+}
+
 // Generic grouped scorer: G <= 4, any M, K.  Table [G][M][K] fp16 in LDS.
 __global__ __launch_bounds__(256) void score_grouped_generic_kernel(
     const uint16_t* __restrict__ lut, int lut_layout, const uint8_t* __restrict__ codes,
@@ -528,6 +643,55 @@ int score_g4_nchunk(int R, int T) {
   return pl.nchunk;
 }
 
+// Stages of 1024 tokens per workgroup of score_any_kernel: the count that takes
+// the fewest rounds of (one table fill + its stages), a fill costing about a
+// stage; slots is the workgroups the chip holds (64 KiB of table per four heads:
+// two per CU up to four heads, one beyond).
+static int any_tok(int R, int T, int G, int cus) {
+  const int64_t slots = (int64_t)cus * (G <= 4 ? 2 : 1);
+  int best = 1;
+  int64_t cost = -1;
+  for (int tok : {1, 2, 4, 8}) {
+    const int64_t wgs = (int64_t)R * ((T + tok * 1024 - 1) / (tok * 1024));
+    const int64_t c = (wgs + slots - 1) / slots * (1 + tok);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = tok;
+    }
+  }
+  return best;
+}
+
+// Scores of any group size from per-head tables (score_any_kernel); outputs as
+// launch_score_g4's.  The caller has checked G <= 8, M = 32, K = 256 and the
+// code rows' alignment (score_g4_supported).
+int launch_score_any(const uint16_t* lut, const uint8_t* codes, int64_t cs_b, int64_t cs_h,
+                     int64_t cs_t, int B, int Hkv, int G, int T, uint16_t* heads, uint16_t* keys,
+                     uint32_t* hist, int key_mode, bool per_head, int cand_start, int cand_end,
+                     const int32_t* plans, int* nchunk_out, hipStream_t st) {
+  DevInfo di;
+  int s = device_info(&di);
+  if (s != LAP_OK) return s;
+  const int R = B * Hkv, tok = any_tok(R, T, G, di.cu_count);
+  const int nchunk = (T + tok * 1024 - 1) / (tok * 1024), hb = G <= 4 ? 1 : 2;
+  const ScoreOut so{heads, keys, hist, key_mode, cand_start, cand_end, plans, per_head ? 1 : 0};
+  const dim3 grid((unsigned)(R * nchunk));
+  const size_t smem = (size_t)hb * kLutBytes +
+                      (hist ? (size_t)(per_head ? G * 2 : 8) * kHPitch * 4 : 0);
+#define LAP_ANY(HB_, PH_)                                                                     \
+  hipLaunchKernelGGL((score_any_kernel<HB_, PH_>), grid, dim3(1024), smem, st, lut, codes,    \
+                     cs_b, cs_h, cs_t, Hkv, G, R, T, tok, so, f16_one())
+  if (hb == 1) {
+    if (per_head) LAP_ANY(1, true); else LAP_ANY(1, false);
+  } else {
+    if (per_head) LAP_ANY(2, true); else LAP_ANY(2, false);
+  }
+#undef LAP_ANY
+  LAP_LAUNCH_CHECK("score_any_kernel");
+  if (nchunk_out) *nchunk_out = nchunk;
+  return LAP_OK;
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 bool score_g4_supported(const uint8_t* codes, int64_t cs_b, int64_t cs_h, int64_t cs_t) {
@@ -559,6 +723,11 @@ extern "C" int lap_lut_score_grouped(const void* lut, int lut_layout, const uint
                            codes_stride_t, 1, Hkv, T, static_cast<uint16_t*>(out), nullptr,
                            nullptr, LAP_KEY_F16, false, 0, 0, nullptr, nullptr, st);
   }
+  if (lut_layout == LAP_LUT_HMK && M == kM && K == kK && aligned16(lut) &&
+      score_g4_supported(codes, 0, codes_stride_h, codes_stride_t))
+    return launch_score_any(L, codes, 0, codes_stride_h, codes_stride_t, 1, Hkv, G, T,
+                            static_cast<uint16_t*>(out), nullptr, nullptr, LAP_KEY_F16, false, 0,
+                            0, nullptr, nullptr, st);
   DevInfo di;
   int s = device_info(&di);
   if (s != LAP_OK) return s;
@@ -587,6 +756,12 @@ extern "C" int lap_lut_score_gqa(const void* lut, const uint8_t* codes, int64_t 
   LAP_CHECK(T >= 0 && N >= 0, "lap_lut_score_gqa: negative size");
   if (!indices) LAP_CHECK(N == T, "lap_lut_score_gqa: dense mode needs N == T");
   if (N == 0) return LAP_OK;
+  if (!indices && G <= 8 && M_start == 0 && M_end == kM && M_stride == kM && K == kK &&
+      aligned16(lut) && score_g4_supported(codes, 0, codes_stride_h, codes_stride_t))
+    return launch_score_any(static_cast<const uint16_t*>(lut), codes, 0, codes_stride_h,
+                            codes_stride_t, 1, Hkv, G, T, static_cast<uint16_t*>(out), nullptr,
+                            nullptr, LAP_KEY_F16, false, 0, 0, nullptr, nullptr,
+                            as_stream(stream));
   DevInfo di;
   int s = device_info(&di);
   if (s != LAP_OK) return s;

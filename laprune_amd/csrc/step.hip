@@ -62,6 +62,11 @@
 namespace lap {
 
 bool score_g4_supported(const uint8_t* codes, int64_t cs_b, int64_t cs_h, int64_t cs_t);
+int retrieve_any(const uint16_t* lut, const uint8_t* codes, int64_t cs_b, int64_t cs_h,
+                 int64_t cs_t, int B, int Hkv, int G, int T, int cand_start, int cand_end, int k,
+                 const lap_row_plan* plans, int k_cols, int key_mode, bool per_head,
+                 void* out_idx, int out_dtype, void* workspace, size_t workspace_bytes,
+                 const char* who, hipStream_t st);
 
 namespace {
 
@@ -1470,10 +1475,17 @@ int decode_step_run(const char* who, const void* lut_gmkg, const uint8_t* codes,
   const int rows = step_rows_per_kv(key_mode, G);
   const int H_idx = Hkv * rows;
   if (G != 4) {
-    // Per-head fp16 scores of every code column (lap_lut_score_gqa over the
-    // [B * Hq][32][256] table), then the top-k of the group max (group
-    // selection) or of each head's row.
-    if (selects) {
+    // The [B * Hq][32][256] table: keys and top-k of the group max (group
+    // selection) or of each head's row.  Code rows that are not 16-byte aligned
+    // take the per-head scorer instead: fp16 scores of every code column
+    // (lap_lut_score_gqa), then their top-k.
+    if (selects && (reinterpret_cast<uintptr_t>(lut_gmkg) & 15) == 0 && codes_stride_t >= kM &&
+        score_g4_supported(codes, codes_stride_b, codes_stride_h, codes_stride_t)) {
+      s = retrieve_any(static_cast<const uint16_t*>(lut_gmkg), codes, codes_stride_b,
+                       codes_stride_h, codes_stride_t, B, Hkv, G, T, cand_start, cand_end, k_eff,
+                       plans, k_cols, km, rows == G, out_idx, idx_dtype, base, cw.ret, who, st);
+      if (s != LAP_OK) return s;
+    } else if (selects) {
       uint16_t* sc = reinterpret_cast<uint16_t*>(base);
       const uint16_t* lut = static_cast<const uint16_t*>(lut_gmkg);
       for (int b = 0; b < B; ++b) {

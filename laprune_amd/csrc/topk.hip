@@ -32,6 +32,10 @@ int launch_score_g4(const uint16_t* lut, bool lut_il, const uint8_t* codes, int6
                     hipStream_t st);
 bool score_g4_supported(const uint8_t* codes, int64_t cs_b, int64_t cs_h, int64_t cs_t);
 int score_g4_nchunk(int R, int T);
+int launch_score_any(const uint16_t* lut, const uint8_t* codes, int64_t cs_b, int64_t cs_h,
+                     int64_t cs_t, int B, int Hkv, int G, int T, uint16_t* heads, uint16_t* keys,
+                     uint32_t* hist, int key_mode, bool per_head, int cand_start, int cand_end,
+                     const int32_t* plans, int* nchunk_out, hipStream_t st);
 
 namespace {
 
@@ -674,20 +678,10 @@ static int retrieve_score_impl(const void* lut_gmkg, const uint8_t* codes, int64
   return LAP_OK;
 }
 
-// Levels over the keys and histograms retrieve_score_impl left, for the
-// B * Hkv * rpk selection rows (rpk as the scorer ran: 1 or 4).
-static int retrieve_select_impl(int B, int Hkv, int rpk, int T, const SelSpec& sp, int n_max,
-                                void* out_idx, int out_dtype, int64_t out_stride,
-                                void* workspace, size_t workspace_bytes, const char* who,
-                                hipStream_t st) {
-  const int R = B * Hkv * rpk;
-  const int C2 = (T + kChunk - 1) / kChunk;
-  Ws w = carve(workspace, R, T, retrieve_chunk_bound(T), C2);
-  LAP_CHECK_CODE(workspace && workspace_bytes >= w.bytes, LAP_ERR_WORKSPACE,
-                 "%s: workspace of %zu bytes needed", who, w.bytes);
-  const int C1 = score_g4_nchunk(B * Hkv, T);  // the scorer's chunks per KV row
-  LAP_CHECK_CODE(C1 > 0 && C1 <= retrieve_chunk_bound(T), LAP_ERR_HIP,
-                 "%s: device query failed", who);
+// Levels over the keys and C1 chunk histograms per row in w, for R selection
+// rows of T columns.
+static int select_from_keys(const Ws& w, int R, int T, int C1, const SelSpec& sp, int n_max,
+                            void* out_idx, int out_dtype, int64_t out_stride, hipStream_t st) {
   const int kpt = row_kernel_kpt(T);
   if (kpt > 0) {
     if (out_dtype == LAP_DTYPE_I64)
@@ -702,6 +696,54 @@ static int retrieve_select_impl(int B, int Hkv, int rpk, int T, const SelSpec& s
   KeySrc ks{w.keys, T, true};
   return run_levels(w, ks, R, sp, n_max, C1, out_idx, out_dtype, out_stride, st);
 }
+
+// The same over what retrieve_score_impl left, for the B * Hkv * rpk selection
+// rows (rpk as the scorer ran: 1 or 4).
+static int retrieve_select_impl(int B, int Hkv, int rpk, int T, const SelSpec& sp, int n_max,
+                                void* out_idx, int out_dtype, int64_t out_stride,
+                                void* workspace, size_t workspace_bytes, const char* who,
+                                hipStream_t st) {
+  const int R = B * Hkv * rpk;
+  const int C2 = (T + kChunk - 1) / kChunk;
+  Ws w = carve(workspace, R, T, retrieve_chunk_bound(T), C2);
+  LAP_CHECK_CODE(workspace && workspace_bytes >= w.bytes, LAP_ERR_WORKSPACE,
+                 "%s: workspace of %zu bytes needed", who, w.bytes);
+  const int C1 = score_g4_nchunk(B * Hkv, T);  // the scorer's chunks per KV row
+  LAP_CHECK_CODE(C1 > 0 && C1 <= retrieve_chunk_bound(T), LAP_ERR_HIP,
+                 "%s: device query failed", who);
+  return select_from_keys(w, R, T, C1, sp, n_max, out_idx, out_dtype, out_stride, st);
+}
+
+namespace lap {
+
+// Scorer and top-k for any group size from per-head tables [B * Hkv * G][32][256]:
+// one selection row per KV row (the group maximum) or, per_head, per query
+// head.  The workspace holds keys and at most T / 1024 histograms per row,
+// which fits where the fp16 scores and lap_topk_select's workspace do.  The
+// caller has checked the arguments and the code rows' alignment.
+int retrieve_any(const uint16_t* lut, const uint8_t* codes, int64_t cs_b, int64_t cs_h,
+                 int64_t cs_t, int B, int Hkv, int G, int T, int cand_start, int cand_end, int k,
+                 const lap_row_plan* plans, int k_cols, int key_mode, bool per_head,
+                 void* out_idx, int out_dtype, void* workspace, size_t workspace_bytes,
+                 const char* who, hipStream_t st) {
+  const int rpk = per_head ? G : 1, R = B * Hkv * rpk;
+  Ws w = carve(workspace, R, T, (T + 1023) / 1024, (T + kChunk - 1) / kChunk);
+  LAP_CHECK_CODE(workspace && workspace_bytes >= w.bytes, LAP_ERR_WORKSPACE,
+                 "%s: workspace of %zu bytes needed", who, w.bytes);
+  int C1 = 0;
+  int s = launch_score_any(lut, codes, cs_b, cs_h, cs_t, B, Hkv, G, T, nullptr, w.keys, w.hist1,
+                           key_mode, per_head, cand_start, cand_end,
+                           reinterpret_cast<const int32_t*>(plans), &C1, st);
+  if (s != LAP_OK) return s;
+  if (plans)
+    return select_from_keys(w, R, T, C1, ragged_spec(plans, Hkv * rpk, k_cols, T), T, out_idx,
+                            out_dtype, k_cols, st);
+  const int n = cand_end - cand_start;
+  return select_from_keys(w, R, T, C1, uniform_spec(cand_start, n, k), n, out_idx, out_dtype, k,
+                          st);
+}
+
+}  // namespace lap
 
 extern "C" int lap_retrieve_score(const void* lut_gmkg, const uint8_t* codes,
                                   int64_t codes_stride_b, int64_t codes_stride_h,
