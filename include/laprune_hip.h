@@ -505,6 +505,24 @@ int lap_rope_append(const void* q, int64_t q_sb, int64_t q_sh,
                     void* cache_v, int64_t cv_sb, int64_t cv_sh, int64_t cv_st,
                     int t_cap, void* q_out, lap_stream_t stream);
 
+/* Element-wise parts of a decode step around the attention layers, rounded to
+ * the model dtype (fp16/bf16) where the model code's tensor ops round.
+ *   lap_rms_norm     out[r] = rnd(w * rnd(x[r] * rsqrt(mean(x[r]^2) + eps))), the
+ *                    mean in fp32; x [rows][H] (row stride given), out contiguous;
+ *                    H and the stride multiples of 8, 16-byte aligned tensors
+ *   lap_silu_mul     out = rnd(rnd(gate / (1 + exp(-gate))) * up), n even elements
+ *   lap_rope_tables  cos, sin [B][2 * half] of pos[b] * inv_freq[i] (fp32), times
+ *                    scaling, both halves alike; inv_freq fp32/fp16/bf16
+ *   lap_argmax_rows  out[r] = first index of row r's largest value (NaN largest) */
+int lap_rms_norm(const void* x, int64_t x_row_stride, int rows, int H, const void* weight,
+                 float eps, int dtype, void* out, lap_stream_t stream);
+int lap_silu_mul(const void* gate, const void* up, int64_t n, int dtype, void* out,
+                 lap_stream_t stream);
+int lap_rope_tables(const int64_t* pos, int B, const void* inv_freq, int freq_dtype, int half,
+                    float scaling, int dtype, void* cos_out, void* sin_out, lap_stream_t stream);
+int lap_argmax_rows(const void* x, int64_t x_row_stride, int rows, int V, int dtype, int64_t* out,
+                    lap_stream_t stream);
+
 /* ======================================================================= *
  * Diagnostics: measurement kernels (no counterpart in the reference; not  *
  * on the path and never called by it).                                    *

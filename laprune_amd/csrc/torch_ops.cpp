@@ -245,6 +245,58 @@ void score_grouped(const at::Tensor& lut, int64_t layout, const at::Tensor& code
         "lap_lut_score_grouped");
 }
 
+// Element-wise parts of a decode step (csrc/model.hip): contiguous tensors of
+// the model dtype.
+void rms_norm(const at::Tensor& x, const at::Tensor& weight, double eps, const at::Tensor& out) {
+  same_gpu("laprune::rms_norm", {&x, &weight, &out});
+  TORCH_CHECK(x.is_contiguous() && out.is_contiguous() && weight.is_contiguous() &&
+                  weight.dim() == 1 && x.size(-1) == weight.numel() && out.sizes() == x.sizes() &&
+                  x.scalar_type() == weight.scalar_type() && out.scalar_type() == x.scalar_type(),
+              "laprune::rms_norm: contiguous x, weight [H] and out of one dtype");
+  const int H = (int)weight.numel();
+  check(lap_rms_norm(ptr(x), H, (int)(x.numel() / H), H, ptr(weight), (float)eps, dtype_code(x),
+                     ptr(out), stream_of(x)),
+        "lap_rms_norm");
+}
+
+void silu_mul(const at::Tensor& gate, const at::Tensor& up, const at::Tensor& out) {
+  same_gpu("laprune::silu_mul", {&gate, &up, &out});
+  TORCH_CHECK(gate.is_contiguous() && up.is_contiguous() && out.is_contiguous() &&
+                  gate.sizes() == up.sizes() && gate.sizes() == out.sizes() &&
+                  gate.scalar_type() == up.scalar_type() &&
+                  out.scalar_type() == gate.scalar_type(),
+              "laprune::silu_mul: contiguous tensors of one shape and dtype");
+  check(lap_silu_mul(ptr(gate), ptr(up), gate.numel(), dtype_code(gate), ptr(out),
+                     stream_of(gate)),
+        "lap_silu_mul");
+}
+
+void rope_tables(const at::Tensor& pos, const at::Tensor& inv_freq, double scaling,
+                 const at::Tensor& cos, const at::Tensor& sin) {
+  same_gpu("laprune::rope_tables", {&pos, &inv_freq, &cos, &sin});
+  const int64_t half = inv_freq.numel();
+  TORCH_CHECK(pos.scalar_type() == at::kLong && pos.is_contiguous() &&
+                  inv_freq.is_contiguous() &&
+                  cos.is_contiguous() && sin.is_contiguous() &&
+                  cos.scalar_type() == sin.scalar_type() &&
+                  cos.numel() == pos.numel() * 2 * half && sin.numel() == cos.numel(),
+              "laprune::rope_tables: pos int64 [B], inv_freq [D/2], cos and sin [B, 1, D]");
+  check(lap_rope_tables(static_cast<const int64_t*>(ptr(pos)), (int)pos.numel(),
+                        ptr(inv_freq), dtype_code(inv_freq), (int)half, (float)scaling,
+                        dtype_code(cos), ptr(cos), ptr(sin), stream_of(cos)),
+        "lap_rope_tables");
+}
+
+void argmax_rows(const at::Tensor& x, const at::Tensor& out) {
+  same_gpu("laprune::argmax_rows", {&x, &out});
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && out.is_contiguous() &&
+                  out.scalar_type() == at::kLong && out.numel() == x.size(0),
+              "laprune::argmax_rows: x [rows, V], out int64 [rows]");
+  check(lap_argmax_rows(ptr(x), x.stride(0), (int)x.size(0), (int)x.size(1), dtype_code(x),
+                        static_cast<int64_t*>(ptr(out)), stream_of(x)),
+        "lap_argmax_rows");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(laprune, m) {
@@ -264,6 +316,11 @@ TORCH_LIBRARY(laprune, m) {
         "Tensor codebooks, Tensor prep, Tensor(a!) codes) -> ()");
   m.def("score_grouped(Tensor lut, int layout, Tensor codes, int G, int M, int K, "
         "Tensor(a!) out) -> ()");
+  m.def("rms_norm(Tensor x, Tensor weight, float eps, Tensor(a!) out) -> ()");
+  m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()");
+  m.def("rope_tables(Tensor pos, Tensor inv_freq, float scaling, Tensor(a!) cos, "
+        "Tensor(b!) sin) -> ()");
+  m.def("argmax_rows(Tensor x, Tensor(a!) out) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(laprune, CUDA, m) {
@@ -274,4 +331,8 @@ TORCH_LIBRARY_IMPL(laprune, CUDA, m) {
   m.impl("rope_append", &rope_append);
   m.impl("encode_keys_ranges", &encode_keys_ranges);
   m.impl("score_grouped", &score_grouped);
+  m.impl("rms_norm", &rms_norm);
+  m.impl("silu_mul", &silu_mul);
+  m.impl("rope_tables", &rope_tables);
+  m.impl("argmax_rows", &argmax_rows);
 }

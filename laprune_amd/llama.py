@@ -29,8 +29,81 @@ import torch
 import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
+from ._ops import ops
 from .cache import DecodeKVCache
 from .retrieval import DenseDecoder, RetrievalConfig, SparseDecoder, check_step_health
+
+
+def _one_token(x: torch.Tensor) -> bool:
+    """Whether x [B, 1, n] is a decode step's activation that the fused
+    element-wise kernels serve; anything else keeps the model's own code."""
+    return (x.dim() == 3 and x.shape[1] == 1 and x.is_cuda and not torch.is_grad_enabled() and
+            x.dtype in (torch.bfloat16, torch.float16) and x.is_contiguous() and
+            x.data_ptr() % 16 == 0 and not torch.compiler.is_compiling())
+
+
+def _fuse_decode_ops(model) -> None:
+    """Single-token forwards of the model's RMSNorms, MLPs and rotary tables
+    as one kernel each where the module is transformers' own class and nobody
+    replaced its forward; other inputs run the class's forward."""
+    from transformers.models.llama import modeling_llama as hf
+
+    def wrap(mod, cls, make):
+        own = mod.__dict__.get("forward")
+        if type(mod) is cls and (own is None or getattr(own, "_lap_decode", False)):
+            f = make(mod)
+            f._lap_decode = True
+            mod.forward = f
+
+    def norm(mod):
+        def forward(hidden_states):
+            x, w = hidden_states, mod.weight
+            if (_one_token(x) and x.shape[-1] % 8 == 0 and w.dtype == x.dtype and
+                    w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0):
+                out = torch.empty_like(x)
+                ops().rms_norm(x, w, mod.variance_epsilon, out)
+                return out
+            return hf.LlamaRMSNorm.forward(mod, x)
+        return forward
+
+    def mlp(mod):
+        def forward(x):
+            if not (_one_token(x) and type(mod.act_fn) in silu):
+                return hf.LlamaMLP.forward(mod, x)
+            g, u = mod.gate_proj(x), mod.up_proj(x)
+            if (_one_token(g) and _one_token(u) and g.dtype == u.dtype and g.shape == u.shape and
+                    g.numel() % 2 == 0):
+                out = torch.empty_like(g)
+                ops().silu_mul(g, u, out)
+            else:
+                out = mod.act_fn(g) * u
+            return mod.down_proj(out)
+        return forward
+
+    def rotary(mod):
+        def forward(x, position_ids):
+            f, p = mod.inv_freq, position_ids
+            if (_one_token(x) and p.dtype == torch.long and p.dim() == 2 and p.shape[1] == 1 and
+                    p.device == x.device and f.device == x.device and p.is_contiguous() and
+                    f.is_contiguous() and 0 < f.numel() <= 128 and
+                    f.dtype in (torch.float32, torch.bfloat16, torch.float16) and
+                    "dynamic" not in mod.rope_type and mod.rope_type != "longrope"):
+                cos = x.new_empty((p.shape[0], 1, 2 * f.numel()))
+                sin = torch.empty_like(cos)
+                ops().rope_tables(p, f, mod.attention_scaling, cos, sin)
+                return cos, sin
+            return hf.LlamaRotaryEmbedding.forward(mod, x, p)
+        return forward
+
+    from transformers.activations import ACT2FN
+    silu = (torch.nn.SiLU, type(ACT2FN["silu"]))
+    m = model.model
+    wrap(m.norm, hf.LlamaRMSNorm, norm)
+    wrap(m.rotary_emb, hf.LlamaRotaryEmbedding, rotary)
+    for layer in m.layers:
+        wrap(layer.input_layernorm, hf.LlamaRMSNorm, norm)
+        wrap(layer.post_attention_layernorm, hf.LlamaRMSNorm, norm)
+        wrap(layer.mlp, hf.LlamaMLP, mlp)
 
 
 @dataclass
@@ -102,6 +175,10 @@ class LAPruneLlama:
             attn = layer.self_attn
             self._fuse_qkv(attn)
             attn.forward = self._make_forward(i, attn)
+        _fuse_decode_ops(model)
+        # every layer's attention ignores the mask; a 4-D one, handed through
+        # as it is, spares a single-token step the launches that build one
+        self._mask = torch.ones((batch, 1, 1, 1), dtype=torch.bool, device=self.dev)
         self._row = None  # sequence being prefilled alone (ragged prefill)
         self.health_every = health_every
         self._since_check = 0
@@ -244,7 +321,9 @@ class LAPruneLlama:
                                "model was wrapped with (wrap it with a larger capacity)")
 
     def _forward(self, ids: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
-        out = self.model(input_ids=ids, position_ids=pos, use_cache=False, logits_to_keep=1)
+        mask = self._mask if ids.shape[1] == 1 else None
+        out = self.model(input_ids=ids, attention_mask=mask, position_ids=pos, use_cache=False,
+                         logits_to_keep=1)
         return out.logits[:, -1]
 
     @torch.no_grad()
@@ -345,7 +424,10 @@ class LAPruneLlama:
         if self._g_logits is None:
             self._g_logits = torch.empty_like(logits)
         self._g_logits.copy_(logits)
-        self._g_next.copy_(logits.argmax(dim=-1, keepdim=True))
+        if logits.dtype in (torch.bfloat16, torch.float16) and logits.stride(-1) == 1:
+            ops().argmax_rows(logits, self._g_next)
+        else:
+            self._g_next.copy_(logits.argmax(dim=-1, keepdim=True))
 
     def _upload_step(self) -> None:
         """Advance every layer's bookkeeping by one token and upload the

@@ -1,0 +1,121 @@
+"""The element-wise kernels of a single-token decode step (RMSNorm, silu * mul,
+rotary tables, argmax) against the model code's own tensor ops, and the
+wrapped modules' route for inputs the kernels do not serve."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.bfloat16, torch.float16]
+
+
+def _ulp_close(got, want, ulps=1):
+    """Equal, or neighbouring values of the dtype: the fp32 values before the
+    rounding differ in the order of a sum or in the last bit of an exp."""
+    i = lambda t: torch.where(t.view(torch.int16) < 0, -32768 - t.view(torch.int16).int(),
+                              t.view(torch.int16).int())
+    assert (i(got) - i(want)).abs().max().item() <= ulps
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H", [8, 72, 4096, 4104, 8192, 8200, 28672])
+def test_rms_norm(dtype, H):
+    from laprune_amd._ops import ops
+    from transformers.models.llama.modeling_llama import LlamaRMSNorm
+    g = torch.Generator(device="cuda").manual_seed(H)
+    m = LlamaRMSNorm(H, eps=1e-5).to("cuda", dtype)
+    with torch.no_grad():
+        m.weight.normal_(1.0, 0.3, generator=g)
+        x = torch.randn((3, 1, H), generator=g, device="cuda").mul(2.5).to(dtype)
+        out = torch.empty_like(x)
+        ops().rms_norm(x, m.weight, m.variance_epsilon, out)
+        # two roundings: a last-bit difference of the first may move the second
+        _ulp_close(out, m(x), 2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [2, 510, 514, 14336])
+def test_silu_mul(dtype, n):
+    from laprune_amd._ops import ops
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a = torch.randn((2, 1, n), generator=g, device="cuda").mul(6).to(dtype)
+    b = torch.randn((2, 1, n), generator=g, device="cuda").to(dtype)
+    a.view(-1)[0] = -math.inf
+    a.view(-1)[1] = math.nan
+    out = torch.empty_like(a)
+    ops().silu_mul(a, b, out)
+    want = torch.nn.functional.silu(a) * b
+    assert torch.equal(out.isnan(), want.isnan())
+    ok = ~want.isnan()
+    _ulp_close(out[ok], want[ok], 2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("freq", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [2, 64, 128, 256])
+def test_rope_tables(dtype, freq, D):
+    from laprune_amd._ops import ops
+    f = (1.0 / 500000.0 ** (torch.arange(0, D, 2, device="cuda").float() / D)).to(freq)
+    pos = torch.tensor([[0], [1], [8191], [131071]], device="cuda")
+    cos = torch.empty((4, 1, D), dtype=dtype, device="cuda")
+    sin = torch.empty_like(cos)
+    ops().rope_tables(pos, f, 1.25, cos, sin)
+    a = (pos.float() * f.float())[:, None]
+    a = torch.cat((a, a), -1)
+    _ulp_close(cos, (a.cos() * 1.25).to(dtype))
+    _ulp_close(sin, (a.sin() * 1.25).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("V,stride", [(1, 1), (7, 9), (8, 8), (8191, 8191), (8193, 8200),
+                                      (128256, 128256)])
+def test_argmax_rows(dtype, V, stride):
+    from laprune_amd._ops import ops
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn((6, stride), generator=g, device="cuda").to(dtype)[:, :V]
+    x[1] = -math.inf
+    x[2] = 0.0
+    x[2, V // 2:] = -0.0
+    x[3, V // 3] = math.nan
+    x[3, V - 1] = math.nan
+    x[4, V // 2:] = 50.0  # ties: the first
+    x[5] = -0.0
+    x[5, V - 1] = 0.0     # equal to -0: the first
+    out = torch.empty((6, 1), dtype=torch.long, device="cuda")
+    ops().argmax_rows(x, out)
+    f = x.cpu().float()
+    want = [next(i for i, v in enumerate(r.tolist())
+                 if (math.isnan(v) if r.isnan().any() else v == r.max().item())) for r in f]
+    assert out[:, 0].tolist() == want
+
+
+def test_wrapped_modules_keep_the_models_code_elsewhere():
+    """Prompt lengths, gradients and fp32 run the class's own forward."""
+    from laprune_amd.llama import _fuse_decode_ops
+    from transformers import LlamaConfig, LlamaForCausalLM
+    torch.manual_seed(0)
+    cfg = LlamaConfig(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1,
+                      num_attention_heads=2, num_key_value_heads=1)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+    L = model.model.layers[0]
+    pos = torch.arange(5, device="cuda")[None]
+    def run(x, p):
+        return [L.input_layernorm(x), L.mlp(x), *model.model.rotary_emb(x, p)]
+    for dt, T, grad in ((torch.bfloat16, 5, False), (torch.bfloat16, 1, True),
+                        (torch.float32, 1, False), (torch.bfloat16, 1, False)):
+        model.to(dt)
+        x = torch.randn((1, T, 64), device="cuda", dtype=dt)
+        with torch.set_grad_enabled(grad):
+            for mod in (L.input_layernorm, L.mlp, model.model.rotary_emb):
+                mod.__dict__.pop("forward", None)
+            want = run(x, pos[:, :T])
+            _fuse_decode_ops(model)
+            got = run(x, pos[:, :T])
+        for a, b in zip(got, want):
+            assert a.dtype == b.dtype and a.requires_grad == b.requires_grad
+            if dt is torch.bfloat16 and T == 1 and not grad:
+                torch.testing.assert_close(a, b, rtol=2 ** -6, atol=2 ** -9)
+            else:
+                assert torch.equal(a, b)
