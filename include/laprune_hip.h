@@ -505,6 +505,15 @@ int lap_rope_append(const void* q, int64_t q_sb, int64_t q_sh,
                     void* cache_v, int64_t cv_sb, int64_t cv_sh, int64_t cv_st,
                     int t_cap, void* q_out, lap_stream_t stream);
 
+/* Projections of one token: lap_gemv out[n] = rnd(sum_k x[k] * w[n][k]), fp32
+ * sums; lap_gemv_glu out[n] = rnd(rnd(g / (1 + exp(-g))) * u) of the rounded sums
+ * g (row n of gate) and u (of up).  x [K], weights [N][K] and out [N] contiguous
+ * fp16 or bf16, x and weights 16-byte aligned, K a multiple of 8. */
+int lap_gemv(const void* x, const void* w, int N, int K, int dtype, void* out,
+             lap_stream_t stream);
+int lap_gemv_glu(const void* x, const void* gate, const void* up, int N, int K, int dtype,
+                 void* out, lap_stream_t stream);
+
 /* Element-wise parts of a decode step around the attention layers, rounded to
  * the model dtype (fp16/bf16) where the model code's tensor ops round.
  *   lap_rms_norm     out[r] = rnd(w * rnd(x[r] * rsqrt(mean(x[r]^2) + eps))), the

@@ -64,6 +64,8 @@ SIGNATURES = {
     "lap_retrieve_select_heads": [i32, i32, i32, i32, i32, i32, vp, i32, vp, sz, vp],
     "lap_rope_append": [vp, i64, i64, vp, i64, i64, vp, i64, i64, vp, vp, i64, i32, i32, i32,
                         i32, i32, vp, vp, i64, i64, i64, vp, i64, i64, i64, i32, vp, vp],
+    "lap_gemv": [vp, vp, i32, i32, i32, vp, vp],
+    "lap_gemv_glu": [vp, vp, vp, i32, i32, i32, vp, vp],
     "lap_rms_norm": [vp, i64, i32, i32, vp, f32, i32, vp, vp],
     "lap_silu_mul": [vp, vp, i64, i32, vp, vp],
     "lap_rope_tables": [vp, i32, vp, i32, i32, f32, i32, vp, vp, vp],

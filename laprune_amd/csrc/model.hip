@@ -6,7 +6,8 @@
 // launches, the rotary tables nine and silu(gate) * up two, some 60 of a
 // two-layer step's 90 (3 to 4 us each inside a captured graph).  With one launch
 // each, and no mask built for one token, that step (2 of Llama-3.1-8B's layers at
-// 32k, weights' and cache's reads 404 us) went from 737 to 549 us.  The arithmetic
+// 32k, weights' and cache's reads 404 us) went from 737 to 549 us
+// (426 with the projections' own kernels).  The arithmetic
 // is that of the model code's tensor ops, rounded to the model dtype where
 // they round (transformers' LlamaRMSNorm, LlamaRotaryEmbedding and LlamaMLP):
 //   rms_norm     rnd(w * rnd(x * rsqrt(mean(x^2) + eps))), the mean in fp32

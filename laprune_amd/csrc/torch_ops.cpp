@@ -259,6 +259,35 @@ void rms_norm(const at::Tensor& x, const at::Tensor& weight, double eps, const a
         "lap_rms_norm");
 }
 
+// Projections of one token (csrc/gemv.hip): x of K elements, w [N][K], out N.
+void gemv(const at::Tensor& x, const at::Tensor& w, const at::Tensor& out) {
+  same_gpu("laprune::gemv", {&x, &w, &out});
+  TORCH_CHECK(x.is_contiguous() && w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
+                  x.numel() == w.size(1) && out.numel() == w.size(0) &&
+                  x.scalar_type() == w.scalar_type() && out.scalar_type() == w.scalar_type() &&
+                  w.size(0) <= INT32_MAX && w.size(1) <= INT32_MAX,
+              "laprune::gemv: contiguous x of K elements, w [N, K], out of N");
+  check(lap_gemv(ptr(x), ptr(w), (int)w.size(0), (int)w.size(1), dtype_code(w), ptr(out),
+                 stream_of(x)),
+        "lap_gemv");
+}
+
+void gemv_glu(const at::Tensor& x, const at::Tensor& gate, const at::Tensor& up,
+              const at::Tensor& out) {
+  same_gpu("laprune::gemv_glu", {&x, &gate, &up, &out});
+  TORCH_CHECK(x.is_contiguous() && gate.dim() == 2 && gate.is_contiguous() &&
+                  up.is_contiguous() && up.sizes() == gate.sizes() && out.is_contiguous() &&
+                  x.numel() == gate.size(1) && out.numel() == gate.size(0) &&
+                  x.scalar_type() == gate.scalar_type() &&
+                  up.scalar_type() == gate.scalar_type() &&
+                  out.scalar_type() == gate.scalar_type() && gate.size(0) <= INT32_MAX &&
+                  gate.size(1) <= INT32_MAX,
+              "laprune::gemv_glu: contiguous x of K elements, gate and up [N, K], out of N");
+  check(lap_gemv_glu(ptr(x), ptr(gate), ptr(up), (int)gate.size(0), (int)gate.size(1),
+                     dtype_code(gate), ptr(out), stream_of(x)),
+        "lap_gemv_glu");
+}
+
 void silu_mul(const at::Tensor& gate, const at::Tensor& up, const at::Tensor& out) {
   same_gpu("laprune::silu_mul", {&gate, &up, &out});
   TORCH_CHECK(gate.is_contiguous() && up.is_contiguous() && out.is_contiguous() &&
@@ -317,6 +346,8 @@ TORCH_LIBRARY(laprune, m) {
   m.def("score_grouped(Tensor lut, int layout, Tensor codes, int G, int M, int K, "
         "Tensor(a!) out) -> ()");
   m.def("rms_norm(Tensor x, Tensor weight, float eps, Tensor(a!) out) -> ()");
+  m.def("gemv(Tensor x, Tensor w, Tensor(a!) out) -> ()");
+  m.def("gemv_glu(Tensor x, Tensor gate, Tensor up, Tensor(a!) out) -> ()");
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()");
   m.def("rope_tables(Tensor pos, Tensor inv_freq, float scaling, Tensor(a!) cos, "
         "Tensor(b!) sin) -> ()");
@@ -332,6 +363,8 @@ TORCH_LIBRARY_IMPL(laprune, CUDA, m) {
   m.impl("encode_keys_ranges", &encode_keys_ranges);
   m.impl("score_grouped", &score_grouped);
   m.impl("rms_norm", &rms_norm);
+  m.impl("gemv", &gemv);
+  m.impl("gemv_glu", &gemv_glu);
   m.impl("silu_mul", &silu_mul);
   m.impl("rope_tables", &rope_tables);
   m.impl("argmax_rows", &argmax_rows);

@@ -42,10 +42,39 @@ def _one_token(x: torch.Tensor) -> bool:
             x.data_ptr() % 16 == 0 and not torch.compiler.is_compiling())
 
 
+def _one_vector(x: torch.Tensor, w: torch.Tensor, b=None) -> bool:
+    """Whether x is one token that the projection kernel serves with weight w."""
+    return (b is None and x.numel() == x.shape[-1] and _one_token(x) and w.dim() == 2 and
+            w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and
+            x.shape[-1] == w.shape[1] and w.shape[1] % 8 == 0 and w.numel() > 0 and
+            w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled(x.device.type))
+
+
+def _linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
+    """F.linear; one token of one sequence goes to the projection kernel."""
+    if _one_vector(x, w, b):
+        out = x.new_empty((1, 1, w.shape[0]))
+        ops().gemv(x, w, out)
+        return out
+    return F.linear(x, w, b)
+
+
+def _plain(mod) -> bool:
+    """A bias-free nn.Linear whose call is its weight's product and no more."""
+    g = torch.nn.modules.module
+    own = mod.__dict__.get("forward")
+    return (type(mod) is torch.nn.Linear and mod.bias is None and
+            (own is None or getattr(own, "_lap_decode", False)) and
+            not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or
+                 mod._backward_pre_hooks or g._global_forward_hooks or
+                 g._global_forward_pre_hooks or g._global_backward_hooks or
+                 g._global_backward_pre_hooks))
+
+
 def _fuse_decode_ops(model) -> None:
-    """Single-token forwards of the model's RMSNorms, MLPs and rotary tables
-    as one kernel each where the module is transformers' own class and nobody
-    replaced its forward; other inputs run the class's forward."""
+    """Single-token forwards of the model's RMSNorms, MLPs, rotary tables and
+    projections as one kernel each where the module is the stock class and
+    nobody replaced its forward; other inputs run the class's forward."""
     from transformers.models.llama import modeling_llama as hf
 
     def wrap(mod, cls, make):
@@ -70,7 +99,13 @@ def _fuse_decode_ops(model) -> None:
         def forward(x):
             if not (_one_token(x) and type(mod.act_fn) in silu):
                 return hf.LlamaMLP.forward(mod, x)
-            g, u = mod.gate_proj(x), mod.up_proj(x)
+            gp, up = mod.gate_proj, mod.up_proj
+            if (_plain(gp) and _plain(up) and gp.weight.shape == up.weight.shape and
+                    _one_vector(x, gp.weight) and _one_vector(x, up.weight)):
+                out = x.new_empty((1, 1, gp.weight.shape[0]))
+                ops().gemv_glu(x, gp.weight, up.weight, out)
+                return mod.down_proj(out)
+            g, u = gp(x), up(x)
             if (_one_token(g) and _one_token(u) and g.dtype == u.dtype and g.shape == u.shape and
                     g.numel() % 2 == 0):
                 out = torch.empty_like(g)
@@ -78,6 +113,11 @@ def _fuse_decode_ops(model) -> None:
             else:
                 out = mod.act_fn(g) * u
             return mod.down_proj(out)
+        return forward
+
+    def linear(mod):
+        def forward(input):
+            return _linear(input, mod.weight, mod.bias)
         return forward
 
     def rotary(mod):
@@ -104,6 +144,10 @@ def _fuse_decode_ops(model) -> None:
         wrap(layer.input_layernorm, hf.LlamaRMSNorm, norm)
         wrap(layer.post_attention_layernorm, hf.LlamaRMSNorm, norm)
         wrap(layer.mlp, hf.LlamaMLP, mlp)
+        for mod in (layer.self_attn.o_proj, layer.mlp.gate_proj, layer.mlp.up_proj,
+                    layer.mlp.down_proj):
+            wrap(mod, torch.nn.Linear, linear)
+    wrap(model.lm_head, torch.nn.Linear, linear)
 
 
 @dataclass
@@ -240,7 +284,7 @@ class LAPruneLlama:
         if f is None:
             return attn.q_proj(h), attn.k_proj(h), attn.v_proj(h)
         w, b, sizes = f
-        return F.linear(h, w, b).split(sizes, dim=-1)
+        return _linear(h, w, b).split(sizes, dim=-1)
 
     def _make_forward(self, idx: int, attn):
         def forward(hidden_states, position_embeddings=None, attention_mask=None,

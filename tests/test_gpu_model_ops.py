@@ -91,6 +91,31 @@ def test_argmax_rows(dtype, V, stride):
     assert out[:, 0].tolist() == want
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K", [(1, 8), (7, 64), (8, 2048), (9, 2056), (1001, 2040),
+                                 (64, 4096), (6, 14336), (4099, 520)])
+def test_gemv(dtype, N, K):
+    """Against the products in 64 bits: the fp32 sum of K exact products errs by
+    at most K * 2^-24 of the sum of their magnitudes, the rounding by half a
+    unit of the dtype; the fused MLP part equals its unfused ops on the
+    kernel's own projections (silu's exp may differ in its last bit)."""
+    from laprune_amd._ops import ops
+    g = torch.Generator(device="cuda").manual_seed(N * 7 + K)
+    x = torch.randn((1, 1, K), generator=g, device="cuda").to(dtype)
+    w = torch.randn((2, N, K), generator=g, device="cuda").mul(0.1).to(dtype)
+    got = torch.empty((2, 1, 1, N), dtype=dtype, device="cuda")
+    for i in range(2):
+        ops().gemv(x, w[i], got[i])
+    want = w.double() @ x.double().view(K)
+    mag = w.double().abs() @ x.double().abs().view(K)
+    half = 2.0 ** (-8 if dtype is torch.bfloat16 else -11)
+    err = (got.view(2, N).double() - want).abs()
+    assert (err <= want.abs() * half + mag * K * 2.0 ** -24 * (1 + half) + 2.0 ** -25).all()
+    glu = torch.empty((1, 1, N), dtype=dtype, device="cuda")
+    ops().gemv_glu(x, w[0], w[1], glu)
+    _ulp_close(glu, torch.nn.functional.silu(got[0]) * got[1], 2)
+
+
 def test_wrapped_modules_keep_the_models_code_elsewhere():
     """Prompt lengths, gradients and fp32 run the class's own forward."""
     from laprune_amd.llama import _fuse_decode_ops
@@ -116,6 +141,7 @@ def test_wrapped_modules_keep_the_models_code_elsewhere():
         for a, b in zip(got, want):
             assert a.dtype == b.dtype and a.requires_grad == b.requires_grad
             if dt is torch.bfloat16 and T == 1 and not grad:
+                # roundings to bf16 of fp32 sums in another order
                 torch.testing.assert_close(a, b, rtol=2 ** -6, atol=2 ** -9)
             else:
                 assert torch.equal(a, b)
