@@ -522,7 +522,8 @@ int lap_gemv_glu(const void* x, const void* gate, const void* up, int N, int K, 
  *   lap_silu_mul     out = rnd(rnd(gate / (1 + exp(-gate))) * up), n even elements
  *   lap_rope_tables  cos, sin [B][2 * half] of pos[b] * inv_freq[i] (fp32), times
  *                    scaling, both halves alike; inv_freq fp32/fp16/bf16
- *   lap_argmax_rows  out[r] = first index of row r's largest value (NaN largest) */
+ *   lap_argmax_rows  out[r] = first index of row r's largest value (NaN largest);
+ *                    copy (may be NULL) [rows][V] receives the rows */
 int lap_rms_norm(const void* x, int64_t x_row_stride, int rows, int H, const void* weight,
                  float eps, int dtype, void* out, lap_stream_t stream);
 int lap_silu_mul(const void* gate, const void* up, int64_t n, int dtype, void* out,
@@ -530,7 +531,7 @@ int lap_silu_mul(const void* gate, const void* up, int64_t n, int dtype, void* o
 int lap_rope_tables(const int64_t* pos, int B, const void* inv_freq, int freq_dtype, int half,
                     float scaling, int dtype, void* cos_out, void* sin_out, lap_stream_t stream);
 int lap_argmax_rows(const void* x, int64_t x_row_stride, int rows, int V, int dtype, int64_t* out,
-                    lap_stream_t stream);
+                    void* copy, lap_stream_t stream);
 
 /* ======================================================================= *
  * Diagnostics: measurement kernels (no counterpart in the reference; not  *

@@ -69,7 +69,7 @@ SIGNATURES = {
     "lap_rms_norm": [vp, i64, i32, i32, vp, f32, i32, vp, vp],
     "lap_silu_mul": [vp, vp, i64, i32, vp, vp],
     "lap_rope_tables": [vp, i32, vp, i32, i32, f32, i32, vp, vp, vp],
-    "lap_argmax_rows": [vp, i64, i32, i32, i32, vp, vp],
+    "lap_argmax_rows": [vp, i64, i32, i32, i32, vp, vp, vp],
     "lap_retrieve_topk_ragged": [vp, vp, i64, i64, i64, i32, i32, i32, vp, i32, i32, vp, vp, i32,
                                  vp, sz, vp],
     "lap_topk_select_ragged": [vp, i64, i32, i32, i32, i32, vp, i32, i32, vp, i32, vp, sz, vp],

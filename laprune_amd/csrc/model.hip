@@ -7,7 +7,7 @@
 // two-layer step's 90 (3 to 4 us each inside a captured graph).  With one launch
 // each, and no mask built for one token, that step (2 of Llama-3.1-8B's layers at
 // 32k, weights' and cache's reads 404 us) went from 737 to 549 us
-// (426 with the projections' own kernels).  The arithmetic
+// (414 with the projections' own kernels and the last touches below).  The arithmetic
 // is that of the model code's tensor ops, rounded to the model dtype where
 // they round (transformers' LlamaRMSNorm, LlamaRotaryEmbedding and LlamaMLP):
 //   rms_norm     rnd(w * rnd(x * rsqrt(mean(x^2) + eps))), the mean in fp32
@@ -140,36 +140,68 @@ __device__ __forceinline__ uint64_t arg_key(uint16_t v, uint32_t i) {
 }
 __device__ __forceinline__ uint64_t max64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// One workgroup per row: 128256 columns are 256 KiB, a few microseconds for
-// one CU; torch's reduction took 40 us.
+// One workgroup per row.  A thread keeps the largest value of its 16-byte
+// vectors and the first vector that holds it, and looks for the element once at
+// the end: 15 instructions per vector; an ordered key per element took 80 and set
+// the time (128256 columns 16.0 us, now 10.2 with the copy).  The step's copy of the logits to the
+// buffer its caller reads rides along (4.7 us as a launch of its own).
 template <int DT>
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t* __restrict__ x,
                                                            int64_t xs, int V,
-                                                           int64_t* __restrict__ out) {
+                                                           int64_t* __restrict__ out,
+                                                           uint16_t* __restrict__ copy) {
   __shared__ uint64_t s_best[16];
   const int tid = threadIdx.x;
   const uint16_t* xr = x + (int64_t)blockIdx.x * xs;
-  uint64_t best = 0;
-  const bool vec = (reinterpret_cast<uintptr_t>(xr) & 15) == 0;
+  uint16_t* cr = copy ? copy + (int64_t)blockIdx.x * V : nullptr;
+  const bool vec = ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(cr)) & 15) == 0;
   const int nv = vec ? V / 8 : 0;
-#pragma unroll 4
-  for (int i = tid; i < nv; i += 1024) {
-    const uint4 v = reinterpret_cast<const uint4*>(xr)[i];
+  const uint4* xv = reinterpret_cast<const uint4*>(xr);
+  float top = -__builtin_inff();
+  int at = tid;
+  auto look = [&](uint4 v, int i) {
     const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+    float m = widen<DT>((uint16_t)u[0]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      best = max64(best, arg_key<DT>((uint16_t)u[e], 8 * i + 2 * e));
-      best = max64(best, arg_key<DT>((uint16_t)(u[e] >> 16), 8 * i + 2 * e + 1));
+    for (int e = 1; e < 8; ++e)
+      m = __builtin_elementwise_maximum(m, widen<DT>((uint16_t)(u[e / 2] >> (16 * (e & 1)))));
+    if (m > top || (m != m && top == top)) {  // ascending vectors: the first is kept
+      top = m;
+      at = i;
+    }
+  };
+  int i = tid;
+#pragma unroll 1
+  for (; i + 7 * 1024 < nv; i += 8 * 1024) {
+    uint4 v[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) v[d] = xv[i + d * 1024];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      look(v[d], i + d * 1024);
+      if (cr) reinterpret_cast<uint4*>(cr)[i + d * 1024] = v[d];
     }
   }
-  for (int i = 8 * nv + tid; i < V; i += 1024) best = max64(best, arg_key<DT>(xr[i], i));
+#pragma unroll 1
+  for (; i < nv; i += 1024) {
+    const uint4 v = xv[i];
+    look(v, i);
+    if (cr) reinterpret_cast<uint4*>(cr)[i] = v;
+  }
+  uint64_t best = 0;
+  if (tid < nv)
+    for (int e = 0; e < 8; ++e) best = max64(best, arg_key<DT>(xr[8 * at + e], 8 * at + e));
+  for (i = 8 * nv + tid; i < V; i += 1024) {
+    best = max64(best, arg_key<DT>(xr[i], i));
+    if (cr) cr[i] = xr[i];
+  }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1)
     best = max64(best, (uint64_t)__shfl_xor((unsigned long long)best, d, 64));
   if ((tid & 63) == 0) s_best[tid >> 6] = best;
   __syncthreads();
   if (tid == 0) {
-    for (int i = 1; i < 16; ++i) best = max64(best, s_best[i]);
+    for (int w = 1; w < 16; ++w) best = max64(best, s_best[w]);
     out[blockIdx.x] = (int64_t)(0xffffffffu - (uint32_t)best);
   }
 }
@@ -240,13 +272,13 @@ extern "C" int lap_rope_tables(const int64_t* pos, int B, const void* inv_freq, 
 }
 
 extern "C" int lap_argmax_rows(const void* x, int64_t x_row_stride, int rows, int V, int dtype,
-                               int64_t* out, lap_stream_t stream) {
+                               int64_t* out, void* copy, lap_stream_t stream) {
   clear_error();
   LAP_CHECK(x && out, "lap_argmax_rows: null pointer");
   LAP_CHECK(dtype == LAP_DTYPE_F16 || dtype == LAP_DTYPE_BF16, "lap_argmax_rows: dtype fp16/bf16");
   LAP_CHECK(rows >= 0 && V > 0 && x_row_stride >= V, "lap_argmax_rows: bad sizes");
   if (rows == 0) return LAP_OK;
   LAP_BY_DTYPE(argmax_rows_kernel, dim3(rows), 1024, static_cast<const uint16_t*>(x), x_row_stride,
-               V, out);
+               V, out, static_cast<uint16_t*>(copy));
   return LAP_OK;
 }

@@ -316,13 +316,18 @@ void rope_tables(const at::Tensor& pos, const at::Tensor& inv_freq, double scali
         "lap_rope_tables");
 }
 
-void argmax_rows(const at::Tensor& x, const at::Tensor& out) {
+void argmax_rows(const at::Tensor& x, const at::Tensor& out,
+                 const std::optional<at::Tensor>& copy) {
   same_gpu("laprune::argmax_rows", {&x, &out});
+  if (copy) same_gpu("laprune::argmax_rows", {&x, &*copy});
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && out.is_contiguous() &&
-                  out.scalar_type() == at::kLong && out.numel() == x.size(0),
-              "laprune::argmax_rows: x [rows, V], out int64 [rows]");
+                  out.scalar_type() == at::kLong && out.numel() == x.size(0) &&
+                  (!copy || (copy->is_contiguous() && copy->sizes() == x.sizes() &&
+                             copy->scalar_type() == x.scalar_type())),
+              "laprune::argmax_rows: x [rows, V], out int64 [rows], copy like x");
   check(lap_argmax_rows(ptr(x), x.stride(0), (int)x.size(0), (int)x.size(1), dtype_code(x),
-                        static_cast<int64_t*>(ptr(out)), stream_of(x)),
+                        static_cast<int64_t*>(ptr(out)), copy ? ptr(*copy) : nullptr,
+                        stream_of(x)),
         "lap_argmax_rows");
 }
 
@@ -351,7 +356,7 @@ TORCH_LIBRARY(laprune, m) {
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()");
   m.def("rope_tables(Tensor pos, Tensor inv_freq, float scaling, Tensor(a!) cos, "
         "Tensor(b!) sin) -> ()");
-  m.def("argmax_rows(Tensor x, Tensor(a!) out) -> ()");
+  m.def("argmax_rows(Tensor x, Tensor(a!) out, Tensor(b!)? copy=None) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(laprune, CUDA, m) {

@@ -441,36 +441,34 @@ class LAPruneLlama:
 
     def _graph_buffers(self):
         B, dev = self.B, self.dev
-        flat = torch.zeros(19 * B, dtype=torch.int32, device=dev)
+        flat = torch.zeros(20 * B, dtype=torch.int32, device=dev)
         self._g_flat = flat
         self._g_plan_sparse = flat[:8 * B].view(B, 8)
         self._g_plan_dense = flat[8 * B:16 * B].view(B, 8)
         self._g_ranges = flat[16 * B:18 * B].view(B, 2)
-        self._g_pos32 = flat[18 * B:].view(B, 1)
-        self._g_pos = torch.zeros((B, 1), dtype=torch.long, device=dev)
+        self._g_pos = flat[18 * B:].view(torch.long).view(B, 1)
         self._q_rope = torch.empty((B, self.Hq, self.D), dtype=self.dtype, device=dev)
         self._g_flush = False
         self._g_tok = torch.zeros((B, 1), dtype=torch.long, device=dev)
         self._g_next = torch.zeros((B, 1), dtype=torch.long, device=dev)
         self._g_logits = None
-        self._g_host = [torch.zeros(19 * B, dtype=torch.int32).pin_memory() for _ in range(4)]
+        self._g_host = [torch.zeros(20 * B, dtype=torch.int32).pin_memory() for _ in range(4)]
         self._g_done = [None] * 4
         self._g_slot = 0
         self._g = True
 
     def _graph_body(self):
-        self._g_pos.copy_(self._g_pos32)
         self._dev_mode = True
         try:
             logits = self._forward(self._g_tok, self._g_pos)
         finally:
             self._dev_mode = False
         if self._g_logits is None:
-            self._g_logits = torch.empty_like(logits)
-        self._g_logits.copy_(logits)
+            self._g_logits = torch.empty_like(logits, memory_format=torch.contiguous_format)
         if logits.dtype in (torch.bfloat16, torch.float16) and logits.stride(-1) == 1:
-            ops().argmax_rows(logits, self._g_next)
+            ops().argmax_rows(logits, self._g_next, self._g_logits)
         else:
+            self._g_logits.copy_(logits)
             self._g_next.copy_(logits.argmax(dim=-1, keepdim=True))
 
     def _upload_step(self) -> None:
@@ -488,7 +486,7 @@ class LAPruneLlama:
         self._g_flush = ranges is not None and any(hi > lo for lo, hi in ranges)
         c0 = next((st for st in self.states if st.sparse is not None), self.states[0])
         t_total = c0.cache.lengths
-        rows = [0] * (19 * B)
+        rows = [0] * (20 * B)  # the last 2 B words are B int64 positions
         if c0.sparse is not None:
             from .retrieval import PLAN_FIELDS
             for b, p in enumerate(c0.sparse.row_plans(c0.cache.encoded_lens, t_total)):
@@ -498,7 +496,7 @@ class LAPruneLlama:
             rows[8 * B + 8 * b:8 * B + 8 * b + 8] = [t, t, 0, 0, 0, 0, 0, t]
             if ranges is not None:
                 rows[16 * B + 2 * b:16 * B + 2 * b + 2] = list(ranges[b])
-            rows[18 * B + b] = pos[b]
+            rows[18 * B + 2 * b] = pos[b]
         i = self._g_slot
         self._g_slot = (i + 1) % len(self._g_host)
         if self._g_done[i] is not None:

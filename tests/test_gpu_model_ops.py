@@ -69,9 +69,11 @@ def test_rope_tables(dtype, freq, D):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("V,stride", [(1, 1), (7, 9), (8, 8), (8191, 8191), (8193, 8200),
-                                      (128256, 128256)])
-def test_argmax_rows(dtype, V, stride):
+@pytest.mark.parametrize("V,stride,copy", [(1, 1, True), (7, 9, False), (8, 8, True),
+                                           (8191, 8191, True), (8193, 8200, False),
+                                           (8200, 8200, True), (65544, 65544, False),
+                                           (128256, 128256, True)])
+def test_argmax_rows(dtype, V, stride, copy):
     from laprune_amd._ops import ops
     g = torch.Generator(device="cuda").manual_seed(V)
     x = torch.randn((6, stride), generator=g, device="cuda").to(dtype)[:, :V]
@@ -84,7 +86,10 @@ def test_argmax_rows(dtype, V, stride):
     x[5] = -0.0
     x[5, V - 1] = 0.0     # equal to -0: the first
     out = torch.empty((6, 1), dtype=torch.long, device="cuda")
-    ops().argmax_rows(x, out)
+    to = torch.full((6, V), 9.0, dtype=dtype, device="cuda") if copy else None
+    ops().argmax_rows(x, out, to)
+    if copy:
+        assert torch.equal(to.view(torch.int16), x.contiguous().view(torch.int16))
     f = x.cpu().float()
     want = [next(i for i, v in enumerate(r.tolist())
                  if (math.isnan(v) if r.isnan().any() else v == r.max().item())) for r in f]
