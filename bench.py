@@ -926,8 +926,8 @@ def main():
             "rows_per_s": round(HKV * ENC_TOKENS / (enc_us * 1e-6), 1),
             "fp32_tflops": round(ENC_FLOP / (enc_us * 1e-6) / 1e12, 3),
             "fp32_peak_tflops": 157.3,
-            "search": "exact fp32 dot16 distances to all 256 entries per stage "
-                      "(encode_exact_kernel, 2 rows per workgroup)",
+            "search": "fp16 MFMA distances to all 256 entries per stage + exact fp32 "
+                      "recheck of uncertain rows (encode_split_kernel, 16 rows per workgroup)",
         },
         "prefill_encode": {
             "workload": "one layer's C4 prefill: 8 KV heads x 131072 post-RoPE key rows "
@@ -938,8 +938,8 @@ def main():
             "rows_per_s": round(PREFILL_ROWS / (pf_ms * 1e-3), 1),
             "search_tflops": round(PREFILL_FLOP / (pf_ms * 1e-3) / 1e12, 2),
             "bf16_mfma_peak_tflops": 2500.0,
-            "search": "bf16 MFMA distances to all 256 entries per stage (the coarse pass) "
-                      "+ exact fp32 recheck of the shortlist (encode_tile_kernel)",
+            "search": "fp16 MFMA distances to all 256 entries per stage + exact fp32 "
+                      "recheck of uncertain rows (encode_wide_kernel)",
         },
         "roofline": {
             "bound": "hbm",
