@@ -1024,6 +1024,14 @@ static bool encode_use_exact(int N, int D, int K) {
   return N <= encode_cus();
 }
 
+// Polls after which a wait of the wide kernel gives up (some 0.1 s; the whole
+// stage takes 6 us).  LAPRUNE_ENCODE_POLLS=n sets it (read at every call).
+static int encode_polls() {
+  const char* e = getenv("LAPRUNE_ENCODE_POLLS");
+  const int n = e ? atoi(e) : -1;
+  return n >= 0 && n < 1 << 20 ? n : 1 << 20;
+}
+
 // Rows whose chunks the wide kernel may read as vectors.
 static bool encode_x_aligned(const RowMap& rm) {
   const int64_t bytes = rm.x_dtype == LAP_DTYPE_F32 ? 16 : 8;
@@ -1039,10 +1047,10 @@ static int launch_wide_as(const RowMap& rm, int N, const float* cb, int M, int K
   const int vec = encode_x_aligned(rm) ? 1 : 0;
   if (K == 256)
     hipLaunchKernelGGL((encode_wide_kernel<D, WAVES, true>), grid, dim3(WAVES * 64), smem, st, rm,
-                       N, cb, M, K, p.wide, p.wstage, p.cn, rnorm, vec);
+                       N, cb, M, K, p.wide, p.wstage, p.cn, rnorm, vec, encode_polls());
   else
     hipLaunchKernelGGL((encode_wide_kernel<D, WAVES, false>), grid, dim3(WAVES * 64), smem, st, rm,
-                       N, cb, M, K, p.wide, p.wstage, p.cn, rnorm, vec);
+                       N, cb, M, K, p.wide, p.wstage, p.cn, rnorm, vec, encode_polls());
   LAP_LAUNCH_CHECK("encode_wide_kernel");
   return LAP_OK;
 }

@@ -263,7 +263,7 @@ template <int D, int WAVES, bool K256>
 __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
     RowMap rm, int N, const float* __restrict__ cb, int M, int K_arg,
     const uint4* __restrict__ wide, const WideStage* __restrict__ stage,
-    const float* __restrict__ cn, float* __restrict__ rnorm, int x_vec) {
+    const float* __restrict__ cn, float* __restrict__ rnorm, int x_vec, int polls) {
   constexpr int KS = D / 16, NV = D / 4;
   constexpr uint32_t kNone = 0x7fffu;
   const int K = K256 ? 256 : K_arg;
@@ -294,17 +294,31 @@ __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
   // of those past the search of one (2, 3), each in turns of WAVES.  A wave
   // asks for stage m + 2 only when all are past the search of stage m, so a
   // counter never mixes two stages.
+  // Waits are bounded, so that the kernel always ends.  A wait that gives up
+  // marks every counter, which ends the waits of the other waves too (each
+  // wave then has in_step false): from there on they neither request nor
+  // count fragments in, so that no stage that is still read is overwritten,
+  // and every row keeps all entries, so that the contract's distances alone
+  // decide and the codes stay what they are.
+  constexpr uint32_t kGaveUp = 0x80000000u;
   __shared__ uint32_t s_cnt[4];
+  bool in_step = true;  // wave-uniform
   auto arrive = [&](int i) {
     if (lane == 0)
       __hip_atomic_fetch_add(&s_cnt[i], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   auto await = [&](int i, uint32_t turns) {
-    for (int spin = 0; spin < (1 << 20); ++spin) {  // bounded: the kernel always ends
-      if (__hip_atomic_load(&s_cnt[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= turns)
-        break;
+    uint32_t v = 0;
+    for (int spin = 0; spin < polls; ++spin) {
+      v = (uint32_t)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(
+          &s_cnt[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      if (v >= turns) break;
       __builtin_amdgcn_s_sleep(1);
     }
+    if (v < turns && lane < 4)
+      __hip_atomic_fetch_or(&s_cnt[lane], kGaveUp, __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_WORKGROUP);
+    in_step = in_step && v >= turns && v < kGaveUp;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
 
@@ -370,7 +384,7 @@ __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
                                       __builtin_fmaf(rns, ws.e2, ws.e0));
 
     // stage 0's fragments came in before the barrier
-    if (m) await(m & 1, (uint32_t)(WAVES * ((m + 1) / 2)));
+    if (m && in_step) await(m & 1, (uint32_t)(WAVES * ((m + 1) / 2)));
 
     // ---- coarse scores, a tile (32 entries) at a time: the lane's running
     // maximum t1 and, per tile, its entries within 2 eps of it.  Step i of a
@@ -451,12 +465,13 @@ __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
     arrive(2 + (m & 1));  // this wave has read stage m's fragments
     if (m + 1 < M) {      // and its share of stage m + 1's is in
       wide_dma_wait();
-      arrive((m + 1) & 1);
+      if (in_step) arrive((m + 1) & 1);
     }
 
     t1 = half_max(t1);
     const float thr = t1 - eps2;
-    const bool all = !(eps2 < 0x1p60f) || !(rns < 0x1p30f);  // outside the fp16 range
+    // outside the fp16 range, or no fragments
+    const bool all = !(eps2 < 0x1p60f) || !(rns < 0x1p30f) || !in_step;
     mk0 = all ? ~0u : mp0 >= thr ? mk0 : 0u;
     mk1 = all ? ~0u : mp1 >= thr ? mk1 : 0u;
     mk2 = all ? ~0u : mp2 >= thr ? mk2 : 0u;
@@ -525,9 +540,9 @@ __global__ __launch_bounds__(WAVES * 64) void encode_wide_kernel(
       rn[u] = wide_dot16<D>(r[u], r[u]);
       if (q == 0 && live[u]) crow[u][m] = (uint8_t)code;
     }
-    if (m + 2 < M) {  // stage m + 2's fragments replace stage m's
+    if (m + 2 < M && in_step) {  // stage m + 2's fragments replace stage m's
       await(2 + (m & 1), (uint32_t)(WAVES * (m / 2 + 1)));
-      request(m + 2);
+      if (in_step) request(m + 2);
     }
   }
 #pragma unroll

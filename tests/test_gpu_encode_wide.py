@@ -84,6 +84,20 @@ def test_out_of_range_rows_and_stages(dev, K, orc, wide):
     _check(K, orc, dev, x, cb, "rows and stages")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("polls", [0, 1, 2])
+def test_waits_that_give_up(dev, K, orc, monkeypatch, polls, M, D):
+    """The wide kernel's waits end after a bounded number of polls.  With a
+    bound that no stage's fragments can meet, or that some waves meet, the
+    contract's distances decide and the codes stay the oracle's."""
+    monkeypatch.setenv("LAPRUNE_ENCODE_TILE", "1")
+    monkeypatch.setenv("LAPRUNE_ENCODE_EXACT", "0")
+    monkeypatch.setenv("LAPRUNE_ENCODE_POLLS", str(polls))
+    x = torch.randn(300, D, generator=gen(polls + M)) * 3
+    _check(K, orc, dev, x, residual_codebooks(23, D, M), f"polls={polls} M={M} D={D}")
+
+
 def test_ties(dev, K, orc, wide):
     """Equal entries, across halves, tiles and pairs of tiles: the lowest wins."""
     cb = residual_codebooks(13)[:5].clone()
