@@ -357,8 +357,14 @@ int lap_sparse_attn_decode_ragged(const void* q, int64_t q_sb, int64_t q_sh,
  * With G = 4 and D = 128, group and per-head selection run as one launch
  * (per KV row, the workgroups of one XCD score, select and attend, and the
  * last merges); other shapes run the kernel chain (G = 4: lap_retrieve_topk;
- * other G: lap_lut_score_gqa of every head, then lap_topk_select (_ragged)
- * over the group max or each head's row; then the sparse attention).
+ * other G: one scorer for up to eight heads that writes the selection keys,
+ * then their top-k, or, where the code rows are not 16-byte aligned,
+ * lap_lut_score_gqa of every head and lap_topk_select (_ragged) over the group
+ * max or each head's row, with the same selection; then the sparse attention).
+ * NaN scores (tables with overflowed entries): a group's key is the largest of
+ * its heads' keys, NaN's with the sign bit clear above and with it set below
+ * all others, for G other than 4; with G = 4 a NaN head is left out of the
+ * group's maximum.
  * Workspace: lap_decode_step_workspace_size
  * with keep_max = k + sink + tail (ragged: k_cols + max_sink + max_tail).  It
  * must be zero-filled once before its first use; every call leaves its

@@ -360,10 +360,21 @@ __global__ __launch_bounds__(1024) void score_any_kernel(
           if (counted) atomicAdd(&s_hist[g * HC * kHPitch + copy + (key >> 8)], 1u);
         }
     } else {
+      // The largest of the heads' keys: that of the largest score, except that
+      // fmaxf drops a NaN, whose key ranks above (or, negative, below) all others
       float mx = fmaxf(fmaxf(e[0][0], e[0][1]), fmaxf(e[0][2], e[0][3]));
-      if constexpr (HB == 2)
+      bool nan = __builtin_isunordered(e[0][0], e[0][1]) || __builtin_isunordered(e[0][2], e[0][3]);
+      if constexpr (HB == 2) {
         mx = fmaxf(mx, fmaxf(fmaxf(e[1][0], e[1][1]), fmaxf(e[1][2], e[1][3])));
-      const uint32_t key = key_of_score(mx, kbf);
+        nan = nan || __builtin_isunordered(e[1][0], e[1][1]) ||
+              __builtin_isunordered(e[1][2], e[1][3]);
+      }
+      uint32_t key = key_of_score(mx, kbf);
+      if (nan) {
+        key = 0;
+#pragma unroll
+        for (int g = 0; g < 4 * HB; ++g) key = max(key, key_of_score(e[g >> 2][g & 3], kbf));
+      }
       so.keys[(int64_t)r * T + t] = (uint16_t)key;
       if (counted) atomicAdd(&s_hist[copy + (key >> 8)], 1u);
     }

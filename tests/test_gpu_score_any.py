@@ -59,3 +59,46 @@ def test_step_selection(dev, G, Hkv, T, k, ragged, select):
         outs.append((o, dec.selected().clone()))
     assert torch.equal(outs[0][1], outs[1][1])
     assert torch.equal(outs[0][0], outs[1][0])
+
+
+@pytest.mark.parametrize("score_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("select", ["group", "head"])
+@pytest.mark.parametrize("G", [1, 3, 7, 8])
+def test_step_selection_with_nan_scores(dev, orc, G, select, score_dtype):
+    """A group's key is the largest of its heads' keys, a NaN head's among them (a
+    positive NaN ranks above every score, a negative one below), whichever path the
+    code rows' alignment takes."""
+    from laprune_amd.retrieval import RetrievalConfig, SparseDecoder
+    print(f"G={G} {select} {score_dtype}", flush=True)
+    Hkv, T, D, k = 2, 3000, 64, 40
+    g = gen(G)
+    lut = (torch.randn(Hkv * G, 32, 256, generator=g) * 0.3).half()
+    codes = torch.randint(0, 255, (1, Hkv, T, 32), generator=g, dtype=torch.uint8)
+    pos = torch.tensor([150, 1023, 1024, 1700, 2047, 2900])
+    neg = torch.tensor([160, 1022, 1025, 2500])
+    lut[:, 0, 255] = float("-inf")       # tokens with entry 255: -inf in every head but
+    lut[G - 1, 0, 255] = float("nan")    # the last of group 0, and the first of group 1
+    lut[G, 0, 255] = float("nan")
+    lut[0, 1, 255] = -torch.tensor(float("nan")).half()
+    codes[:, :, pos, 0] = 255
+    codes[:, :, neg, 1] = 255
+    q = torch.randn(1, Hkv * G, 1, D, generator=g).bfloat16().to(dev)
+    kk = torch.randn(1, Hkv, T, D, generator=g).bfloat16().to(dev)
+    odd = torch.zeros(1, Hkv, T, 33, dtype=torch.uint8, device=dev)
+    odd[..., :32] = codes.to(dev)
+    cfg = RetrievalConfig(topk=k, select=select, score_dtype=score_dtype)
+    got = []
+    for c in (codes.to(dev), odd[..., :32]):
+        dec = SparseDecoder(gaussian_codebooks(3, D).to(dev), 1, Hkv * G, Hkv, D, T, cfg)
+        dec.lut.copy_(lut)
+        p = dec.plan(T, T)
+        dec.last_k = p["k"]
+        dec._decode_step(q[:, :, 0], c, kk, kk, T, T, p, None, 0, 0, 0)
+        got.append(dec.selected()[0].cpu().numpy())
+    assert np.array_equal(got[0], got[1])
+    s = orc.score_grouped(lut.numpy().view(np.uint16), codes[0].numpy(), G)
+    want = orc.topk(s, k, 1 if select == "head" else G, p["cand_start"], p["cand_end"],
+                    key_bf16=score_dtype == torch.bfloat16)
+    assert np.array_equal(got[0], want)
+    if select == "group":
+        assert np.isin(pos.numpy(), got[0][0]).all() and np.isin(pos.numpy(), got[0][1]).all()
