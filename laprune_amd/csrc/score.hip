@@ -767,7 +767,13 @@ extern "C" int lap_lut_score_gqa(const void* lut, const uint8_t* codes, int64_t 
   LAP_CHECK(T >= 0 && N >= 0, "lap_lut_score_gqa: negative size");
   if (!indices) LAP_CHECK(N == T, "lap_lut_score_gqa: dense mode needs N == T");
   if (N == 0) return LAP_OK;
-  if (!indices && G <= 8 && M_start == 0 && M_end == kM && M_stride == kM && K == kK &&
+  // Few tokens of more than four heads keep one head per workgroup: the 128 KiB
+  // fill of score_any_kernel's tables takes longer than their lookups (us in a
+  // captured loop, per head / eight heads per pass: G = 8, 1 row of 4096 tokens
+  // 6.1 / 7.2, 2 x 16384 7.3 / 7.4, 1 x 49152 7.9 / 7.4; G = 5, 8 x 4096 7.1 / 7.2,
+  // 4 x 16384 7.8 / 7.3; up to 512 tokens a row 6.0 / 5.6).
+  const bool few = G > 4 && T > 768 && (int64_t)Hkv * T <= 32768;
+  if (!indices && G <= 8 && !few && M_start == 0 && M_end == kM && M_stride == kM && K == kK &&
       aligned16(lut) && score_g4_supported(codes, 0, codes_stride_h, codes_stride_t))
     return launch_score_any(static_cast<const uint16_t*>(lut), codes, 0, codes_stride_h,
                             codes_stride_t, 1, Hkv, G, T, static_cast<uint16_t*>(out), nullptr,
