@@ -121,6 +121,17 @@ def test_gemv(dtype, N, K):
     _ulp_close(glu, torch.nn.functional.silu(got[0]) * got[1], 2)
 
 
+@pytest.mark.parametrize("N,K,own", [(8192, 64, True), (8200, 64, False), (151936, 384, False),
+                                     (8200, 512, True), (64, 8, True)])
+def test_short_rows_keep_the_librarys_product(N, K, own):
+    """The projection kernel takes one token where it is the faster one."""
+    from laprune_amd.llama import _one_vector
+    x = torch.zeros((1, 1, K), dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros((N, K), dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        assert _one_vector(x, w) == own
+
+
 def test_wrapped_modules_keep_the_models_code_elsewhere():
     """Prompt lengths, gradients and fp32 run the class's own forward."""
     from laprune_amd.llama import _fuse_decode_ops
