@@ -22,8 +22,10 @@ downloads anything (build it from a local ``LlamaConfig``).
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass, field
+from types import MethodType
 
 import torch
 import torch.nn.functional as F
@@ -63,16 +65,85 @@ def _linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
     return F.linear(x, w, b)
 
 
+def _own_forward(mod) -> bool:
+    """Whether mod runs its class's forward (unpickled modules hold it bound) or the
+    one bound to it here, and not a replacement (one that wraps either included)."""
+    f = mod.__dict__.get("forward")
+    return f is None or (isinstance(f, MethodType) and f.__self__ is mod and
+                         (f.__func__ in _DECODE_FORWARDS or f.__func__ is type(mod).forward))
+
+
 def _plain(mod) -> bool:
     """A bias-free nn.Linear whose call is its weight's product and no more."""
     g = torch.nn.modules.module
-    own = mod.__dict__.get("forward")
-    return (type(mod) is torch.nn.Linear and mod.bias is None and
-            (own is None or getattr(own, "_lap_decode", False)) and
+    return (type(mod) is torch.nn.Linear and mod.bias is None and _own_forward(mod) and
             not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or
                  mod._backward_pre_hooks or g._global_forward_hooks or
                  g._global_forward_pre_hooks or g._global_backward_hooks or
                  g._global_backward_pre_hooks))
+
+
+# Single-token forwards, bound to the modules as methods: a deep copy of a module
+# runs on its own weights, and a pickled one finds its class's forward (hence the
+# name).  Other inputs run the class's forward.
+
+def _norm_forward(self, hidden_states):
+    x, w = hidden_states, self.weight
+    if (_one_token(x) and x.shape[-1] % 8 == 0 and w.dtype == x.dtype and
+            w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0):
+        out = torch.empty_like(x)
+        ops().rms_norm(x, w, self.variance_epsilon, out)
+        return out
+    return type(self).forward(self, x)
+
+
+def _mlp_forward(self, x):
+    if not (_one_token(x) and type(self.act_fn) in _silu_types()):
+        return type(self).forward(self, x)
+    gp, up = self.gate_proj, self.up_proj
+    if (_plain(gp) and _plain(up) and gp.weight.shape == up.weight.shape and
+            _one_vector(x, gp.weight) and _one_vector(x, up.weight)):
+        out = x.new_empty((1, 1, gp.weight.shape[0]))
+        ops().gemv_glu(x, gp.weight, up.weight, out)
+        return self.down_proj(out)
+    g, u = gp(x), up(x)
+    if (_one_token(g) and _one_token(u) and g.dtype == u.dtype and g.shape == u.shape and
+            g.numel() % 2 == 0):
+        out = torch.empty_like(g)
+        ops().silu_mul(g, u, out)
+    else:
+        out = self.act_fn(g) * u
+    return self.down_proj(out)
+
+
+def _linear_forward(self, input):
+    return _linear(input, self.weight, self.bias)
+
+
+def _rotary_forward(self, x, position_ids):
+    f, p = self.inv_freq, position_ids
+    if (_one_token(x) and p.dtype == torch.long and p.dim() == 2 and p.shape[1] == 1 and
+            p.device == x.device and f.device == x.device and p.is_contiguous() and
+            f.is_contiguous() and 0 < f.numel() <= 128 and
+            f.dtype in (torch.float32, torch.bfloat16, torch.float16) and
+            "dynamic" not in self.rope_type and self.rope_type != "longrope"):
+        cos = x.new_empty((p.shape[0], 1, 2 * f.numel()))
+        sin = torch.empty_like(cos)
+        ops().rope_tables(p, f, self.attention_scaling, cos, sin)
+        return cos, sin
+    return type(self).forward(self, x, p)
+
+
+_DECODE_FORWARDS = (_norm_forward, _mlp_forward, _linear_forward, _rotary_forward)
+for _f in _DECODE_FORWARDS:
+    _f.__name__ = "forward"
+del _f
+
+
+@functools.lru_cache(None)
+def _silu_types() -> tuple:
+    from transformers.activations import ACT2FN
+    return torch.nn.SiLU, type(ACT2FN["silu"])
 
 
 def _fuse_decode_ops(model) -> None:
@@ -81,77 +152,21 @@ def _fuse_decode_ops(model) -> None:
     nobody replaced its forward; other inputs run the class's forward."""
     from transformers.models.llama import modeling_llama as hf
 
-    def wrap(mod, cls, make):
-        own = mod.__dict__.get("forward")
-        if type(mod) is cls and (own is None or getattr(own, "_lap_decode", False)):
-            f = make(mod)
-            f._lap_decode = True
-            mod.forward = f
+    def wrap(mod, cls, forward):
+        if type(mod) is cls and _own_forward(mod):
+            mod.forward = MethodType(forward, mod)
 
-    def norm(mod):
-        def forward(hidden_states):
-            x, w = hidden_states, mod.weight
-            if (_one_token(x) and x.shape[-1] % 8 == 0 and w.dtype == x.dtype and
-                    w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0):
-                out = torch.empty_like(x)
-                ops().rms_norm(x, w, mod.variance_epsilon, out)
-                return out
-            return hf.LlamaRMSNorm.forward(mod, x)
-        return forward
-
-    def mlp(mod):
-        def forward(x):
-            if not (_one_token(x) and type(mod.act_fn) in silu):
-                return hf.LlamaMLP.forward(mod, x)
-            gp, up = mod.gate_proj, mod.up_proj
-            if (_plain(gp) and _plain(up) and gp.weight.shape == up.weight.shape and
-                    _one_vector(x, gp.weight) and _one_vector(x, up.weight)):
-                out = x.new_empty((1, 1, gp.weight.shape[0]))
-                ops().gemv_glu(x, gp.weight, up.weight, out)
-                return mod.down_proj(out)
-            g, u = gp(x), up(x)
-            if (_one_token(g) and _one_token(u) and g.dtype == u.dtype and g.shape == u.shape and
-                    g.numel() % 2 == 0):
-                out = torch.empty_like(g)
-                ops().silu_mul(g, u, out)
-            else:
-                out = mod.act_fn(g) * u
-            return mod.down_proj(out)
-        return forward
-
-    def linear(mod):
-        def forward(input):
-            return _linear(input, mod.weight, mod.bias)
-        return forward
-
-    def rotary(mod):
-        def forward(x, position_ids):
-            f, p = mod.inv_freq, position_ids
-            if (_one_token(x) and p.dtype == torch.long and p.dim() == 2 and p.shape[1] == 1 and
-                    p.device == x.device and f.device == x.device and p.is_contiguous() and
-                    f.is_contiguous() and 0 < f.numel() <= 128 and
-                    f.dtype in (torch.float32, torch.bfloat16, torch.float16) and
-                    "dynamic" not in mod.rope_type and mod.rope_type != "longrope"):
-                cos = x.new_empty((p.shape[0], 1, 2 * f.numel()))
-                sin = torch.empty_like(cos)
-                ops().rope_tables(p, f, mod.attention_scaling, cos, sin)
-                return cos, sin
-            return hf.LlamaRotaryEmbedding.forward(mod, x, p)
-        return forward
-
-    from transformers.activations import ACT2FN
-    silu = (torch.nn.SiLU, type(ACT2FN["silu"]))
     m = model.model
-    wrap(m.norm, hf.LlamaRMSNorm, norm)
-    wrap(m.rotary_emb, hf.LlamaRotaryEmbedding, rotary)
+    wrap(m.norm, hf.LlamaRMSNorm, _norm_forward)
+    wrap(m.rotary_emb, hf.LlamaRotaryEmbedding, _rotary_forward)
     for layer in m.layers:
-        wrap(layer.input_layernorm, hf.LlamaRMSNorm, norm)
-        wrap(layer.post_attention_layernorm, hf.LlamaRMSNorm, norm)
-        wrap(layer.mlp, hf.LlamaMLP, mlp)
+        wrap(layer.input_layernorm, hf.LlamaRMSNorm, _norm_forward)
+        wrap(layer.post_attention_layernorm, hf.LlamaRMSNorm, _norm_forward)
+        wrap(layer.mlp, hf.LlamaMLP, _mlp_forward)
         for mod in (layer.self_attn.o_proj, layer.mlp.gate_proj, layer.mlp.up_proj,
                     layer.mlp.down_proj):
-            wrap(mod, torch.nn.Linear, linear)
-    wrap(model.lm_head, torch.nn.Linear, linear)
+            wrap(mod, torch.nn.Linear, _linear_forward)
+    wrap(model.lm_head, torch.nn.Linear, _linear_forward)
 
 
 @dataclass
