@@ -156,17 +156,31 @@ def _fuse_decode_ops(model) -> None:
         if type(mod) is cls and _own_forward(mod):
             mod.forward = MethodType(forward, mod)
 
+    def part(mod, name):  # None: a model without it (another MLP, no rotary module)
+        return getattr(mod, name, None)
+
     m = model.model
-    wrap(m.norm, hf.LlamaRMSNorm, _norm_forward)
-    wrap(m.rotary_emb, hf.LlamaRotaryEmbedding, _rotary_forward)
+    wrap(part(m, "norm"), hf.LlamaRMSNorm, _norm_forward)
+    wrap(part(m, "rotary_emb"), hf.LlamaRotaryEmbedding, _rotary_forward)
     for layer in m.layers:
-        wrap(layer.input_layernorm, hf.LlamaRMSNorm, _norm_forward)
-        wrap(layer.post_attention_layernorm, hf.LlamaRMSNorm, _norm_forward)
-        wrap(layer.mlp, hf.LlamaMLP, _mlp_forward)
-        for mod in (layer.self_attn.o_proj, layer.mlp.gate_proj, layer.mlp.up_proj,
-                    layer.mlp.down_proj):
+        wrap(part(layer, "input_layernorm"), hf.LlamaRMSNorm, _norm_forward)
+        wrap(part(layer, "post_attention_layernorm"), hf.LlamaRMSNorm, _norm_forward)
+        mlp = part(layer, "mlp")
+        wrap(mlp, hf.LlamaMLP, _mlp_forward)
+        for mod in (part(layer.self_attn, "o_proj"), part(mlp, "gate_proj"),
+                    part(mlp, "up_proj"), part(mlp, "down_proj")):
             wrap(mod, torch.nn.Linear, _linear_forward)
-    wrap(model.lm_head, torch.nn.Linear, _linear_forward)
+    wrap(part(model, "lm_head"), torch.nn.Linear, _linear_forward)
+
+
+def _step_mask(model, batch: int, device):
+    """Attention mask of a single-token forward.  Every layer's attention ignores
+    it; a 4-D one, which LlamaModel hands through as it is, spares the step the
+    launches that build one.  Another model class gets none, as for a prompt."""
+    from transformers.models.llama import modeling_llama as hf
+    if type(model.model) is not hf.LlamaModel:
+        return None
+    return torch.ones((batch, 1, 1, 1), dtype=torch.bool, device=device)
 
 
 @dataclass
@@ -239,9 +253,7 @@ class LAPruneLlama:
             self._fuse_qkv(attn)
             attn.forward = self._make_forward(i, attn)
         _fuse_decode_ops(model)
-        # every layer's attention ignores the mask; a 4-D one, handed through
-        # as it is, spares a single-token step the launches that build one
-        self._mask = torch.ones((batch, 1, 1, 1), dtype=torch.bool, device=self.dev)
+        self._mask = _step_mask(model, batch, self.dev)
         self._row = None  # sequence being prefilled alone (ragged prefill)
         self.health_every = health_every
         self._since_check = 0

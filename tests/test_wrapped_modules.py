@@ -65,3 +65,24 @@ def test_a_replaced_forward_stays(fused):
     assert gate.forward is outer
     fused.model.layers[0].mlp(torch.randn(1, 1, 32))
     assert calls
+
+
+def test_models_without_some_part_are_served():
+    """Only the attention layers' projections are needed: another MLP, norms of
+    other names, no rotary module and no head are left as they are."""
+    from laprune_amd.llama import _fuse_decode_ops, _step_mask
+    model = _model()
+    assert _step_mask(model, 2, "cpu").shape == (2, 1, 1, 1)
+    layer = model.model.layers[0]
+    layer.mlp = torch.nn.Sequential(torch.nn.Linear(32, 48), torch.nn.Linear(48, 32))
+    del model.model.rotary_emb, model.model.norm, layer.input_layernorm, model.lm_head
+    _fuse_decode_ops(model)
+    assert "forward" in layer.self_attn.o_proj.__dict__
+    del layer.mlp, layer.self_attn.o_proj
+    _fuse_decode_ops(model)
+
+    class Other(type(model.model)):
+        pass
+
+    model.model.__class__ = Other
+    assert _step_mask(model, 2, "cpu") is None
