@@ -73,14 +73,20 @@ def _own_forward(mod) -> bool:
                          (f.__func__ in _DECODE_FORWARDS or f.__func__ is type(mod).forward))
 
 
-def _plain(mod) -> bool:
-    """A bias-free nn.Linear whose call is its weight's product and no more."""
+def _unhooked(mod) -> bool:
+    """Whether a call of mod is its class's forward and no more: the fused MLP
+    leaves such a call out."""
     g = torch.nn.modules.module
-    return (type(mod) is torch.nn.Linear and mod.bias is None and _own_forward(mod) and
+    return (_own_forward(mod) and
             not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or
                  mod._backward_pre_hooks or g._global_forward_hooks or
                  g._global_forward_pre_hooks or g._global_backward_hooks or
                  g._global_backward_pre_hooks))
+
+
+def _plain(mod) -> bool:
+    """A bias-free nn.Linear whose call is its weight's product and no more."""
+    return type(mod) is torch.nn.Linear and mod.bias is None and _unhooked(mod)
 
 
 # Single-token forwards, bound to the modules as methods: a deep copy of a module
@@ -98,7 +104,7 @@ def _norm_forward(self, hidden_states):
 
 
 def _mlp_forward(self, x):
-    if not (_one_token(x) and type(self.act_fn) in _silu_types()):
+    if not (_one_token(x) and type(self.act_fn) in _silu_types() and _unhooked(self.act_fn)):
         return type(self).forward(self, x)
     gp, up = self.gate_proj, self.up_proj
     if (_plain(gp) and _plain(up) and gp.weight.shape == up.weight.shape and

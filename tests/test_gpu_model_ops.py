@@ -161,3 +161,35 @@ def test_wrapped_modules_keep_the_models_code_elsewhere():
                 torch.testing.assert_close(a, b, rtol=2 ** -6, atol=2 ** -9)
             else:
                 assert torch.equal(a, b)
+
+
+def _layer(I=96):
+    from laprune_amd.llama import _fuse_decode_ops
+    from transformers import LlamaConfig, LlamaForCausalLM
+    torch.manual_seed(0)
+    cfg = LlamaConfig(vocab_size=64, hidden_size=64, intermediate_size=I, num_hidden_layers=1,
+                      num_attention_heads=2, num_key_value_heads=1)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+    _fuse_decode_ops(model)
+    return model.model.layers[0]
+
+
+@pytest.mark.parametrize("B", [1, 3])
+def test_hooks_on_the_activation_run(B):
+    """The fused MLP leaves the activation's call out, unless something waits for it
+    or stands in its place."""
+    x = torch.randn((B, 1, 64), device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        mlp, seen = _layer().mlp, []
+        h = mlp.act_fn.register_forward_hook(lambda m, i, o: seen.append(o) or 2 * o)
+        want = mlp.down_proj(2 * torch.nn.functional.silu(mlp.gate_proj(x)) * mlp.up_proj(x))
+        assert torch.equal(mlp(x), want) and len(seen) == 1
+        h.remove()
+        mlp.act_fn.forward = lambda t: 0 * t
+        assert not mlp(x).any()
+        del mlp.act_fn.forward
+        h = torch.nn.modules.module.register_module_forward_hook(
+            lambda m, i, o: seen.append(m) if m is mlp.act_fn else None)
+        mlp(x)
+        h.remove()
+        assert seen[-1] is mlp.act_fn
