@@ -29,6 +29,7 @@ from types import MethodType
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from ._ops import ops
@@ -36,12 +37,28 @@ from .cache import DecodeKVCache
 from .retrieval import DenseDecoder, RetrievalConfig, SparseDecoder, check_step_health
 
 
+def _unwatched() -> bool:
+    """Whether the calling ops only have to compute: no gradient, compiler, trace,
+    function transform (vmap, jvp), forward-mode level or dispatch mode (fake
+    tensors, op counters) looks at them, all of which a kernel call would pass by."""
+    return not (torch.compiler.is_compiling() or torch.is_grad_enabled() or
+                forward_ad._current_level >= 0 or
+                torch._C._functorch.peek_interpreter_stack() is not None or
+                torch._C._len_torch_dispatch_stack() or
+                torch._C._get_tracing_state() is not None)
+
+
+def _plain_tensor(x: torch.Tensor) -> bool:
+    """A tensor of no other class, contiguous and aligned to 16 bytes."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and x.is_contiguous() and
+            x.data_ptr() % 16 == 0)
+
+
 def _one_token(x: torch.Tensor) -> bool:
     """Whether x [B, 1, n] is a decode step's activation that the fused
     element-wise kernels serve; anything else keeps the model's own code."""
-    return (x.dim() == 3 and x.shape[1] == 1 and x.is_cuda and not torch.is_grad_enabled() and
-            x.dtype in (torch.bfloat16, torch.float16) and x.is_contiguous() and
-            x.data_ptr() % 16 == 0 and not torch.compiler.is_compiling())
+    return (_unwatched() and x.dim() == 3 and x.shape[1] == 1 and x.is_cuda and
+            x.dtype in (torch.bfloat16, torch.float16) and _plain_tensor(x))
 
 
 def _one_vector(x: torch.Tensor, w: torch.Tensor, b=None) -> bool:
@@ -50,10 +67,10 @@ def _one_vector(x: torch.Tensor, w: torch.Tensor, b=None) -> bool:
     kernel, bf16: 14336 x 64 4.4 / 4.6, 32000 x 256 8.2 / 8.7, 151936 x 384 34.3 / 35.4;
     8192 x 64 4.2 / 3.2, and from 512 columns on the kernel at every height)."""
     return (b is None and x.numel() == x.shape[-1] and _one_token(x) and w.dim() == 2 and
-            w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and
-            x.shape[-1] == w.shape[1] and w.shape[1] % 8 == 0 and w.numel() > 0 and
+            w.dtype == x.dtype and w.device == x.device and x.shape[-1] == w.shape[1] and
+            w.shape[1] % 8 == 0 and w.numel() > 0 and _plain_tensor(w) and
             (w.shape[1] >= 512 or w.shape[0] <= 8192) and
-            w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled(x.device.type))
+            not torch.is_autocast_enabled(x.device.type))
 
 
 def _linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
@@ -96,7 +113,7 @@ def _plain(mod) -> bool:
 def _norm_forward(self, hidden_states):
     x, w = hidden_states, self.weight
     if (_one_token(x) and x.shape[-1] % 8 == 0 and w.dtype == x.dtype and
-            w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0):
+            w.device == x.device and _plain_tensor(w)):
         out = torch.empty_like(x)
         ops().rms_norm(x, w, self.variance_epsilon, out)
         return out
@@ -130,7 +147,8 @@ def _rotary_forward(self, x, position_ids):
     f, p = self.inv_freq, position_ids
     if (_one_token(x) and p.dtype == torch.long and p.dim() == 2 and p.shape[1] == 1 and
             p.device == x.device and f.device == x.device and p.is_contiguous() and
-            f.is_contiguous() and 0 < f.numel() <= 128 and
+            f.is_contiguous() and type(p) is torch.Tensor and type(f) is torch.Tensor and
+            0 < f.numel() <= 128 and
             f.dtype in (torch.float32, torch.bfloat16, torch.float16) and
             "dynamic" not in self.rope_type and self.rope_type != "longrope"):
         cos = x.new_empty((p.shape[0], 1, 2 * f.numel()))

@@ -5,6 +5,7 @@ import math
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 pytestmark = pytest.mark.gpu
 
@@ -193,3 +194,65 @@ def test_hooks_on_the_activation_run(B):
         mlp(x)
         h.remove()
         assert seen[-1] is mlp.act_fn
+
+
+def _calls(layer, x):
+    yield from (lambda t: layer.mlp(t), lambda t: layer.input_layernorm(t),
+                lambda t: layer.self_attn.o_proj(t))
+
+
+@pytest.mark.parametrize("B", [1, 3])
+def test_forward_mode_tangents_pass_through(B):
+    layer = _layer()
+    x, t = torch.randn((2, B, 1, 64), device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        for f in _calls(layer, x):
+            with forward_ad.dual_level():
+                got = forward_ad.unpack_dual(f(forward_ad.make_dual(x, t)))
+            want = torch.func.jvp(f, (x,), (t,))
+            assert torch.equal(got.primal, want[0]) and torch.equal(got.tangent, want[1])
+            assert got.tangent.any()
+
+
+def test_vmap_passes_through():
+    layer = _layer()
+    xs = torch.randn((5, 1, 1, 64), device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        for f in _calls(layer, xs):
+            got = torch.vmap(f)(xs)
+            # bf16 results of fp32 sums in another order
+            torch.testing.assert_close(got, torch.stack([f(x) for x in xs]), rtol=2 ** -6,
+                                       atol=2 ** -9)
+
+
+def test_modes_and_traces_see_the_models_ops():
+    from torch.utils.flop_counter import FlopCounterMode
+    layer = _layer().requires_grad_(False)
+    x = torch.randn((1, 1, 64), device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        with FlopCounterMode(display=False) as c:
+            layer.mlp(x)
+        assert c.get_total_flops() == 3 * 2 * 64 * 96
+        traced = torch.jit.trace(lambda t: layer.mlp(t), x, check_trace=False)
+        assert "laprune::" not in str(traced.graph)
+
+
+def test_weights_of_another_class_keep_their_product():
+    class Doubled(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            plain = [a.as_subclass(torch.Tensor) if isinstance(a, Doubled) else a for a in args]
+            out = func(*plain, **(kwargs or {}))
+            return 2 * out if func is torch.nn.functional.linear else out
+
+    layer = _layer()
+    x = torch.randn((1, 1, 64), device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        for mod in (layer.self_attn.o_proj, layer.mlp.gate_proj):
+            w = mod.weight.detach()
+            del mod.weight
+            mod.weight = w.as_subclass(Doubled)
+            assert torch.equal(mod(x), 2 * torch.nn.functional.linear(x, w))
+        g, u = mod(x), layer.mlp.up_proj(x)
+        torch.testing.assert_close(layer.mlp(x), layer.mlp.down_proj(
+            torch.nn.functional.silu(g) * u), rtol=2 ** -6, atol=2 ** -9)
