@@ -250,7 +250,8 @@ void score_grouped(const at::Tensor& lut, int64_t layout, const at::Tensor& code
 void rms_norm(const at::Tensor& x, const at::Tensor& weight, double eps, const at::Tensor& out) {
   same_gpu("laprune::rms_norm", {&x, &weight, &out});
   TORCH_CHECK(x.is_contiguous() && out.is_contiguous() && weight.is_contiguous() &&
-                  weight.dim() == 1 && x.size(-1) == weight.numel() && out.sizes() == x.sizes() &&
+                  weight.dim() == 1 && weight.numel() > 0 && x.dim() > 0 &&
+                  x.size(-1) == weight.numel() && out.sizes() == x.sizes() &&
                   x.scalar_type() == weight.scalar_type() && out.scalar_type() == x.scalar_type(),
               "laprune::rms_norm: contiguous x, weight [H] and out of one dtype");
   const int H = (int)weight.numel();

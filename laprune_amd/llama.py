@@ -57,7 +57,7 @@ def _plain_tensor(x: torch.Tensor) -> bool:
 def _one_token(x: torch.Tensor) -> bool:
     """Whether x [B, 1, n] is a decode step's activation that the fused
     element-wise kernels serve; anything else keeps the model's own code."""
-    return (_unwatched() and x.dim() == 3 and x.shape[1] == 1 and x.is_cuda and
+    return (_unwatched() and x.dim() == 3 and x.shape[1] == 1 and x.numel() > 0 and x.is_cuda and
             x.dtype in (torch.bfloat16, torch.float16) and _plain_tensor(x))
 
 

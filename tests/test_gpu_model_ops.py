@@ -36,6 +36,21 @@ def test_rms_norm(dtype, H):
         _ulp_close(out, m(x), 2)
 
 
+def test_rms_norm_of_no_columns_is_refused():
+    from laprune_amd._ops import ops
+    x, w = (torch.empty(s, dtype=torch.bfloat16, device="cuda") for s in ((2, 1, 0), (0,)))
+    with pytest.raises(RuntimeError, match="rms_norm"):
+        ops().rms_norm(x, w, 1e-5, torch.empty_like(x))
+
+
+def test_empty_batches_run_the_models_code():
+    layer = _layer()
+    x = torch.empty((0, 1, 64), dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        for f in _calls(layer, x):
+            assert f(x).shape == x.shape
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n", [2, 510, 514, 14336])
 def test_silu_mul(dtype, n):
