@@ -29,3 +29,14 @@ def orc():
     from oracle import orc as o
     o.lib()
     return o
+
+
+@pytest.fixture
+def form(request, monkeypatch):
+    """Forces an encode kernel of _forms.KERNELS; its head dim."""
+    kernel, D = request.param
+    monkeypatch.setenv("LAPRUNE_ENCODE_TILE", "1" if kernel == "wide" else "0")
+    monkeypatch.setenv("LAPRUNE_ENCODE_EXACT", "1" if kernel == "exact" else "0")
+    if kernel.startswith("split"):
+        monkeypatch.setenv("LAPRUNE_ENCODE_ROWS", kernel[5:])
+    return D

@@ -9,6 +9,8 @@ import numpy as np
 import pytest
 import torch
 
+from _forms import encode_forms
+
 pytestmark = pytest.mark.gpu
 
 
@@ -502,9 +504,9 @@ def test_dense_attn_decode(dev, K, orc, T):
 
 # --------------------------------------------------------------- A6 encode
 
-# 20000 and 40000 rows take the 32- and 64-row workgroup tiles (two and four
-# row groups sharing each codebook fragment) on a 256-CU device; 40003 leaves a
-# partial last tile.
+# 512 and 20000 rows take the split kernel with 16 and 32 rows per workgroup, 37 the
+# exact one, 3 the head dim 256's, 40000 the wide one on a 256-CU device; 40003
+# leaves a partial last wave.
 @pytest.mark.parametrize("N,D", [(512, 128), (37, 64), (3, 256), (20000, 128), (40003, 128),
                                  (40000, 64)])
 def test_encode_bit_exact(dev, K, orc, N, D):
@@ -525,7 +527,8 @@ def test_encode_bit_exact(dev, K, orc, N, D):
     assert np.array_equal(rn.cpu().numpy()[rows].view(np.uint32), want_r.view(np.uint32))
 
 
-def test_encode_c3_config(dev, K, orc, encode_rows):
+@encode_forms(128)
+def test_encode_c3_config(dev, K, orc, form):
     """BASELINE config C3 exactly: 8 KV heads x 64 post-RoPE keys (pre-RoPE
     bf16 N(0,1) x per-channel U(0.5, 4), rotate-half RoPE with theta 500000
     at positions 131008..131071), 32 x 256 fp32 codebooks N(0, 0.02):
@@ -549,22 +552,11 @@ def test_encode_c3_config(dev, K, orc, encode_rows):
     assert np.array_equal(rn.cpu().numpy().view(np.uint32), want_r.view(np.uint32))
 
 
-@pytest.fixture(params=["4", "16", "x1", "x2"])
-def encode_rows(request, monkeypatch):
-    """Runs a test on the 4-row and the 16-row MFMA workgroup kernels and on
-    the exact-distance kernel at 1 and 2 rows per workgroup (flushes take
-    the exact kernel by default)."""
-    if request.param.startswith("x"):
-        monkeypatch.setenv("LAPRUNE_ENCODE_EXACT", "1")
-        monkeypatch.setenv("LAPRUNE_ENCODE_EXACT_ROWS", request.param[1:])
-        return int(request.param[1:])
-    monkeypatch.setenv("LAPRUNE_ENCODE_ROWS", request.param)
-    return int(request.param)
-
-
-@pytest.mark.parametrize("N,D", [(512, 128), (37, 64), (2048, 128)])
-def test_encode_both_small_kernels(dev, K, orc, N, D, encode_rows):
+@encode_forms(64, 128, 256)
+@pytest.mark.parametrize("N", [37, 512, 2048])
+def test_encode_kernels(dev, K, orc, N, form):
     g = _gen(150 + N)
+    D = form
     M, Kc = 32, 256
     x = torch.randn(N, D, generator=g) * (torch.rand(D, generator=g) * 3.5 + 0.5)
     cb = torch.randn(M, Kc, D, generator=g) * 0.02
@@ -575,10 +567,12 @@ def test_encode_both_small_kernels(dev, K, orc, N, D, encode_rows):
     assert np.array_equal(rn.cpu().numpy().view(np.uint32), want_r.view(np.uint32))
 
 
-@pytest.mark.parametrize("Kc,D", [(60, 64), (48, 128), (16, 64), (240, 128)])
-def test_encode_bit_exact_entry_counts(dev, K, orc, Kc, D, encode_rows):
-    """K % 16 != 0 takes the all-VALU search, the rest the MFMA search with
-    fewer entry tiles than waves."""
+@encode_forms(64, 128, 256)
+@pytest.mark.parametrize("Kc", [16, 48, 60, 240])
+def test_encode_bit_exact_entry_counts(dev, K, orc, Kc, form):
+    """Fewer entry tiles than waves; at head dim 256, K % 16 != 0 takes the VALU
+    search."""
+    D = form
     g = _gen(120 + Kc)
     M, N = 8, 45
     x = torch.randn(N, D, generator=g) * 2.0
@@ -590,11 +584,12 @@ def test_encode_bit_exact_entry_counts(dev, K, orc, Kc, D, encode_rows):
     assert np.array_equal(rn.cpu().numpy().view(np.uint32), want_r.view(np.uint32))
 
 
-def test_encode_more_stages_than_staged_codes(dev, K, orc, encode_rows):
-    """M = 80 stages: codes of stages 64 and up are stored as they are
-    chosen, the first 64 staged in LDS and stored at the end."""
+@encode_forms(64, 128, 256)
+def test_encode_more_stages_than_staged_codes(dev, K, orc, form):
+    """M = 80 stages: codes of stages 64 (split kernel: 32) and up are stored as
+    they are chosen, the first ones staged in LDS and stored at the end."""
     g = _gen(125)
-    M, Kc, D, N = 80, 32, 64, 45
+    M, Kc, D, N = 80, 32, form, 45
     x = torch.randn(N, D, generator=g) * 2.0
     cb = torch.randn(M, Kc, D, generator=g) * 0.05
     codes, rn = K.aq_encode_greedy(x.to(dev), cb.to(dev))
@@ -605,12 +600,13 @@ def test_encode_more_stages_than_staged_codes(dev, K, orc, encode_rows):
     assert np.array_equal(rn.cpu().numpy().view(np.uint32), want_r.view(np.uint32))
 
 
-def test_encode_ties_and_near_ties(dev, K, orc, encode_rows):
+@encode_forms(64, 128, 256)
+def test_encode_ties_and_near_ties(dev, K, orc, form):
     """Duplicate entries (exact ties: the lowest index must win) and entries a
-    few ulps apart, far inside the bf16 coarse error, so the exact recheck
+    few ulps apart, far inside the coarse searches' error, so the exact recheck
     decides."""
     g = _gen(130)
-    M, Kc, D, N = 6, 64, 128, 80
+    M, Kc, D, N = 6, 64, form, 80
     cb = torch.randn(M, Kc, D, generator=g) * 0.05
     cb[:, 40] = cb[:, 7]                       # exact duplicate of an earlier entry
     cb[:, 41] = cb[:, 7] * (1 + 2 ** -20)      # a hair away from it
@@ -629,12 +625,13 @@ def test_encode_ties_and_near_ties(dev, K, orc, encode_rows):
     assert 40 not in set(codes.cpu().numpy().ravel().tolist())  # ties go to entry 7
 
 
-def test_encode_non_finite_rows(dev, K, orc, encode_rows):
+@encode_forms(64, 128, 256)
+def test_encode_non_finite_rows(dev, K, orc, form):
     """Rows whose norms overflow or hold NaN take the full exact scan and
     follow the contract (NaN and +inf distances never win; no finite
     distance gives code 0)."""
     g = _gen(140)
-    M, Kc, D, N = 4, 32, 64, 20
+    M, Kc, D, N = 4, 32, form, 20
     cb = torch.randn(M, Kc, D, generator=g) * 0.05
     x = torch.randn(N, D, generator=g)
     x[3, 5] = float("nan")

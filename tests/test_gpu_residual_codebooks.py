@@ -4,14 +4,14 @@ near 9-10; tests/_synth.residual_codebooks) instead of N(0, 0.02).
 
 Covered bit for bit against the oracle: the LUT builder (both forms, fp32 and
 fp16 codebooks), the fused G = 4 scorer on codes that real keys produce, the
-greedy encode on all three kernels (4-row, 16-row and 64-row workgroups), the
-codebook manager's serving methods, and the one-launch decode step's
-selection.  The fp16 table's range is checked too (no entry overflows).
+greedy encode on all its kernels, the codebook manager's serving methods, and
+the one-launch decode step's selection.  The fp16 table's range is checked too (no entry overflows).
 """
 import numpy as np
 import pytest
 import torch
 
+from _forms import encode_forms
 from _synth import c3_keys, residual_codebooks
 
 pytestmark = pytest.mark.gpu
@@ -81,27 +81,23 @@ def test_score_residual_codebooks_real_codes(dev, K, orc, cb):
     print(f"stage-0 entries used: {int((used > 0).sum())} of 256")
 
 
-@pytest.mark.parametrize("which", ["4", "16", "x1", "x2"])
-def test_encode_residual_codebooks(dev, K, orc, cb, which, monkeypatch):
-    """C3-shaped keys (norms about 28) against residual codebooks, on the
-    4-row and the 16-row MFMA workgroup kernels and the exact-distance one."""
-    if which.startswith("x"):
-        monkeypatch.setenv("LAPRUNE_ENCODE_EXACT", "1")
-        monkeypatch.setenv("LAPRUNE_ENCODE_EXACT_ROWS", which[1:])
-    else:
-        monkeypatch.setenv("LAPRUNE_ENCODE_ROWS", which)
-    x = c3_keys(45)
+@encode_forms(64, 128, 256)
+def test_encode_residual_codebooks(dev, K, orc, form):
+    """C3-shaped keys (norms about 28 at head dim 128) against residual codebooks,
+    on every encode kernel."""
+    cb = residual_codebooks(41, form)
+    x = c3_keys(45, D=form)
     codes, rn = K.aq_encode_greedy(x.to(dev), cb.to(dev))
     torch.cuda.synchronize()
     want_c, want_r = orc.encode(x.numpy(), cb.numpy())
     assert np.array_equal(codes.cpu().numpy(), want_c)
     assert np.array_equal(rn.cpu().numpy().view(np.uint32), want_r.view(np.uint32))
-    print(f"rows {which}: mean residual norm {float(want_r.mean()):.3f} "
+    print(f"D = {form}: mean residual norm {float(want_r.mean()):.3f} "
           f"of key norm {float(np.linalg.norm(x.numpy(), axis=1).mean()):.3f}")
 
 
 def test_encode_residual_codebooks_large_launch(dev, K, orc, cb):
-    """40,000 rows take the 64-row workgroup kernel; sampled rows checked."""
+    """40,000 rows take the wide kernel on a 256-CU device; sampled rows checked."""
     g = torch.Generator().manual_seed(46)
     N = 40000
     x = (torch.randn(N, D, generator=g) * (torch.rand(D, generator=g) * 3.5 + 0.5))
