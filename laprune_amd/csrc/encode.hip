@@ -273,12 +273,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 template <int D>
 struct EncCfg {
-  static constexpr int KS = D / 16;             // MFMA k-steps per tile
-  static constexpr int TPW = D == 256 ? 2 : 4;  // N-tiles per wave
-  static constexpr int WAVES = 16 / TPW;        // covers K <= 256 (16 tiles)
+  static constexpr int KS = D / 16;       // MFMA k-steps per tile
+  static constexpr int TPW = 2;           // N-tiles per wave
+  static constexpr int WAVES = 16 / TPW;  // covers K <= 256 (16 tiles)
   static constexpr int THREADS = WAVES * 64;
-  static constexpr int L = D / 16;              // dot16 chain length
-  static constexpr int CAP = D == 256 ? 2 : 4;  // exact rechecks loaded per batch
+  static constexpr int L = D / 16;        // dot16 chain length
+  static constexpr int CAP = 2;           // exact rechecks loaded per batch
 };
 
 __global__ __launch_bounds__(256) void encode_prep_frag(const float* __restrict__ cb, int M,
@@ -553,8 +553,8 @@ __device__ __forceinline__ void enc_stage(EncShared<D>& s, const EncStage<D>& st
     // Batches of CAP survivors: all their loads are issued before any
     // is used, so a batch costs one memory latency.
     for (uint32_t base = 0; base < n; base += C::CAP) {
-      const uint32_t word = C::CAP == 4 ? *reinterpret_cast<const uint32_t*>(&s.list[row][base])
-                                        : *reinterpret_cast<const uint16_t*>(&s.list[row][base]);
+      static_assert(C::CAP == 2, "a batch's entries in one 16-bit read");
+      const uint32_t word = *reinterpret_cast<const uint16_t*>(&s.list[row][base]);
       int kq[C::CAP];
       float c[C::CAP][C::L], cnk[C::CAP];
 #pragma unroll
