@@ -249,7 +249,7 @@ __device__ __forceinline__ void wide_dma(const uint4* src, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %0, off"
                :
                : "v"(src), "s"(dst)
-               : "memory");
+               : "memory", "m0");
 }
 __device__ __forceinline__ void wide_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
