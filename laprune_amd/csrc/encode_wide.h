@@ -32,9 +32,11 @@
 //   |A_k - A*_k| <= s d' + (2^-11 s + sqrt(D) (2^-14 + 2^-25)) (c' + d')  fp16 inputs
 //                 + (D + 16) 2^-23 (s c' + h)                      fp32 MFMA sums
 //                 + 20 2^-24 s c' + 2^-24 (2^b rn + 2 h + s c')    E_k's own rounding
-// (2^-14: subnormal fp16 inputs may be flushed; the sum term takes one ulp of
-// the largest magnitude per addition, in any order).  eps is above the sum,
-// with 2^-15 for the (D + 16) 2^-23 and 2^-22 for rn's 2^-24, and an entry with
+//                 + min(h, 2^-8) (1 + 2^-10) + 2^-19               the parts of h'
+// (2^-14: subnormal fp16 inputs may be flushed, of the parts of h' / 64 less than
+// 2^-14 in all; the sum term takes one ulp of the largest magnitude per addition,
+// in any order).  eps is above the sum, with 2^-15 for the (D + 16) 2^-23, 2^-22
+// for rn's 2^-24 and 2^-18 for the last, and an entry with
 // A_k < max A - 2 eps cannot attain the minimum of E, nor tie with it.  Stages
 // or rows outside the fp16 range (norms that are not finite, codebook norms
 // past 2^12, rows past 2^15) keep every entry.  With post-RoPE keys and
@@ -122,7 +124,8 @@ __global__ __launch_bounds__(1024) void encode_prep_wide(const float* __restrict
     WideStage w;
     w.e1 = 2.05f * (d_ + (0x1p-11f + 0x1p-15f + 0x1p-17f) * (c + d_));
     w.e0 = bad ? INFINITY
-               : 2.05f * (sqrtf((float)D) * 0x1.01p-14f * (c + d_) + 0x1p-15f * h + 0x1p-18f);
+               : 2.05f * (sqrtf((float)D) * 0x1.01p-14f * (c + d_) + 0x1p-15f * h + 0x1p-18f +
+                          1.01f * fminf(h, 0x1p-8f));
     w.e2 = 2.05f * sc * 0x1p-22f;
     w.pad = 0.f;
     stage[m] = w;
