@@ -29,6 +29,8 @@ _ops = None
 def ops():
     """``torch.ops.laprune`` after loading the binding (raises if it is not built)."""
     global _ops
+    if _ops is not None:  # set once, after the load
+        return _ops
     with _lock:
         if _ops is None:
             if not LIB_PATH.exists():

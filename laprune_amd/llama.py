@@ -37,15 +37,18 @@ from .cache import DecodeKVCache
 from .retrieval import DenseDecoder, RetrievalConfig, SparseDecoder, check_step_health
 
 
+# looked up once: every wrapped call of an eager step asks them
+_compiling, _grad_on = torch.compiler.is_compiling, torch.is_grad_enabled
+_transforms, _modes = torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_dispatch_stack
+_trace = torch._C._get_tracing_state
+
+
 def _unwatched() -> bool:
-    """Whether the calling ops only have to compute: no gradient, compiler, trace,
-    function transform (vmap, jvp), forward-mode level or dispatch mode (fake
-    tensors, op counters) looks at them, all of which a kernel call would pass by."""
-    return not (torch.compiler.is_compiling() or torch.is_grad_enabled() or
-                forward_ad._current_level >= 0 or
-                torch._C._functorch.peek_interpreter_stack() is not None or
-                torch._C._len_torch_dispatch_stack() or
-                torch._C._get_tracing_state() is not None)
+    """Whether the calling ops only have to compute: no compiler, gradient, function
+    transform (vmap, jvp), forward-mode level, dispatch mode (fake tensors, op
+    counters) or trace looks at them, all of which a kernel call would pass by."""
+    return not (_compiling() or _grad_on() or forward_ad._current_level >= 0 or
+                _transforms() is not None or _modes() or _trace() is not None)
 
 
 def _plain_tensor(x: torch.Tensor) -> bool:
@@ -61,16 +64,21 @@ def _one_token(x: torch.Tensor) -> bool:
             x.dtype in (torch.bfloat16, torch.float16) and _plain_tensor(x))
 
 
-def _one_vector(x: torch.Tensor, w: torch.Tensor, b=None) -> bool:
-    """Whether x is one token that the projection kernel serves with weight w, and
-    serves faster: many short rows are the library's (us in a captured loop, library /
-    kernel, bf16: 14336 x 64 4.4 / 4.6, 32000 x 256 8.2 / 8.7, 151936 x 384 34.3 / 35.4;
-    8192 x 64 4.2 / 3.2, and from 512 columns on the kernel at every height)."""
-    return (b is None and x.numel() == x.shape[-1] and _one_token(x) and w.dim() == 2 and
-            w.dtype == x.dtype and w.device == x.device and x.shape[-1] == w.shape[1] and
-            w.shape[1] % 8 == 0 and w.numel() > 0 and _plain_tensor(w) and
-            (w.shape[1] >= 512 or w.shape[0] <= 8192) and
+def _weight_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the projection kernel serves weight w with the tokens of x, and faster
+    than the library: many short rows are the library's (us in a captured loop,
+    library / kernel, bf16: 14336 x 64 4.4 / 4.6, 32000 x 256 8.2 / 8.7, 151936 x 384
+    34.3 / 35.4; 8192 x 64 4.2 / 3.2, and from 512 columns on the kernel at every
+    height)."""
+    return (w.dim() == 2 and w.dtype == x.dtype and w.device == x.device and
+            x.shape[-1] == w.shape[1] and w.shape[1] % 8 == 0 and w.numel() > 0 and
+            _plain_tensor(w) and (w.shape[1] >= 512 or w.shape[0] <= 8192) and
             not torch.is_autocast_enabled(x.device.type))
+
+
+def _one_vector(x: torch.Tensor, w: torch.Tensor, b=None) -> bool:
+    """Whether x is one token for the projection kernel with weight w."""
+    return b is None and _one_token(x) and x.numel() == x.shape[-1] and _weight_fits(x, w)
 
 
 def _linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
@@ -124,8 +132,9 @@ def _mlp_forward(self, x):
     if not (_one_token(x) and type(self.act_fn) in _silu_types() and _unhooked(self.act_fn)):
         return type(self).forward(self, x)
     gp, up = self.gate_proj, self.up_proj
-    if (_plain(gp) and _plain(up) and gp.weight.shape == up.weight.shape and
-            _one_vector(x, gp.weight) and _one_vector(x, up.weight)):
+    if (x.numel() == x.shape[-1] and _plain(gp) and _plain(up) and
+            gp.weight.shape == up.weight.shape and _weight_fits(x, gp.weight) and
+            _weight_fits(x, up.weight)):
         out = x.new_empty((1, 1, gp.weight.shape[0]))
         ops().gemv_glu(x, gp.weight, up.weight, out)
         return self.down_proj(out)
