@@ -149,27 +149,31 @@ def test_short_rows_keep_the_librarys_product(N, K, own):
 
 
 def test_wrapped_modules_keep_the_models_code_elsewhere():
-    """Prompt lengths, gradients and fp32 run the class's own forward."""
+    """Prompt lengths, gradients and fp32 run the class's own forward; the expected
+    values come from a copy that was never wrapped."""
+    import copy
     from laprune_amd.llama import _fuse_decode_ops
     from transformers import LlamaConfig, LlamaForCausalLM
     torch.manual_seed(0)
     cfg = LlamaConfig(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1,
                       num_attention_heads=2, num_key_value_heads=1)
     model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
-    L = model.model.layers[0]
+    plain = copy.deepcopy(model)
+    _fuse_decode_ops(model)
     pos = torch.arange(5, device="cuda")[None]
-    def run(x, p):
-        return [L.input_layernorm(x), L.mlp(x), *model.model.rotary_emb(x, p)]
+
+    def run(m, x, p):
+        layer = m.model.layers[0]
+        return [layer.input_layernorm(x), layer.mlp(x), layer.self_attn.o_proj(x), m.lm_head(x),
+                *m.model.rotary_emb(x, p)]
+
     for dt, T, grad in ((torch.bfloat16, 5, False), (torch.bfloat16, 1, True),
                         (torch.float32, 1, False), (torch.bfloat16, 1, False)):
-        model.to(dt)
+        model.to(dt), plain.to(dt)
+        assert not any("forward" in m.__dict__ for m in plain.modules())
         x = torch.randn((1, T, 64), device="cuda", dtype=dt)
         with torch.set_grad_enabled(grad):
-            for mod in (L.input_layernorm, L.mlp, model.model.rotary_emb):
-                mod.__dict__.pop("forward", None)
-            want = run(x, pos[:, :T])
-            _fuse_decode_ops(model)
-            got = run(x, pos[:, :T])
+            want, got = run(plain, x, pos[:, :T]), run(model, x, pos[:, :T])
         for a, b in zip(got, want):
             assert a.dtype == b.dtype and a.requires_grad == b.requires_grad
             if dt is torch.bfloat16 and T == 1 and not grad:
