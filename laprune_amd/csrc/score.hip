@@ -771,8 +771,8 @@ extern "C" int lap_lut_score_gqa(const void* lut, const uint8_t* codes, int64_t 
   // fill of score_any_kernel's tables takes longer than their lookups (us in a
   // captured loop, per head / eight heads per pass: G = 8, 1 row of 4096 tokens
   // 6.1 / 7.2, 2 x 16384 7.3 / 7.4, 1 x 49152 7.9 / 7.4; G = 5, 8 x 4096 7.1 / 7.2,
-  // 4 x 16384 7.8 / 7.3; up to 512 tokens a row 6.0 / 5.6).
-  const bool few = G > 4 && T > 768 && (int64_t)Hkv * T <= 32768;
+  // 4 x 16384 7.8 / 7.3; 512 tokens a row 6.0 / 5.6, 768 6.0 / 6.4).
+  const bool few = G > 4 && T > 512 && (int64_t)Hkv * T <= 32768;
   if (!indices && G <= 8 && !few && M_start == 0 && M_end == kM && M_stride == kM && K == kK &&
       aligned16(lut) && score_g4_supported(codes, 0, codes_stride_h, codes_stride_t))
     return launch_score_any(static_cast<const uint16_t*>(lut), codes, 0, codes_stride_h,

@@ -21,7 +21,7 @@ def K(dev):
     (1, 8, 1), (2, 3, 1023), (3, 2, 1024), (3, 2, 1025), (5, 1, 2049), (6, 4, 40000),
     (7, 8, 33333), (8, 2, 5000), (8, 8, 131073), (1, 8, 131073), (4, 2, 1500),
     # more than four heads: both sides of the sizes that keep one head per workgroup
-    (8, 3, 1), (5, 1, 768), (5, 1, 769), (7, 33, 1023), (6, 32, 1024), (8, 32, 1025),
+    (8, 3, 1), (5, 1, 512), (5, 1, 513), (7, 33, 1023), (6, 32, 1024), (8, 32, 1025),
     (5, 16, 2049), (8, 1, 32768), (8, 1, 32769)])
 def test_scores(dev, K, orc, G, Hkv, T):
     print(f"G={G} Hkv={Hkv} T={T}", flush=True)
