@@ -5,7 +5,7 @@
   ``_decode_attention`` calls (aq_evaluation.py:165): the fp16 LUT from
   ``lap_lut_build`` (fp32 fmaf chain over d, RNE to fp16) summed by the
   grouped scorer (``lap_lut_score_grouped``, sequential fp32 over m, fp16
-  out) for G <= 4, or by the per-head GQA scorer for larger groups.
+  out) for G <= 4, or by ``lap_lut_score_gqa`` for larger groups.
 * ``approx_inner_product_multihead`` (:519-630): per-head codes, the same LUT
   summed by the MHA scorer; ``approx_inner_product`` (:459-520) is its
   one-query form with the head's group codebooks.

@@ -16,8 +16,10 @@
 // an fp16 residual and an argmax of r.c - |c|^2/2; the fp32 path is the one
 // followed here.
 //
-// lap_encode_prepare builds, once per codebook: Ct[m][d][k] (the codebook
-// transposed so that lane-contiguous k is memory-contiguous) and cn[m][k].
+// lap_encode_prepare builds, once per codebook: cn[m][k] and its square root, the
+// tables of the kernel that serves the shape (struct Prep) and Ct[m][d][k] (the
+// codebook transposed so that lane-contiguous k is memory-contiguous: the VALU
+// form's, which by default serves D = 256 with K % 16 != 0 alone).
 // encode_greedy_kernel (the VALU form): one wave per row; lane l owns entries
 // k = 4l..4l+3 and keeps their 16 chain sums in registers while d streams
 // through; the row's residual lives in LDS and is read as a broadcast.
@@ -990,10 +992,12 @@ static int encode_cus() {
 
 // D = 64 and 128 (encode_wide.h).  More than 128 rows per CU: the wide kernel,
 // a wave per 32 rows; up to there the split kernel, whose stage is shorter but
-// which reads the stage's table for every 32 rows instead of 256 (D = 128, us:
-// 16384 rows 93 split, 32768 rows 179 split and 190-210 wide, 65536 rows 355
-// split and 230 wide; the 16- and 4-row bf16 kernels that they replaced took 90
-// for 2048 rows, 327 for 16384).
+// which reads the stage's table for every 32 rows instead of 256.  us, split /
+// wide, rows of magnitude 2: D = 128, 16384 rows 107 / 190, 32768 187 / 190, 40000
+// 218 / 191, 65536 330 / 226, 131072 653 / 441; D = 64, 32768 120 / 143, 40000
+// 142 / 144, 65536 217 / 154.  The wide kernel's time comes in rounds of 256 rows
+// per CU: just past a round (65600 rows 353 / 381, at D = 64 227 / 258; 81920 at
+// D = 64 269 / 282) the split kernel would be faster still.
 // LAPRUNE_ENCODE_TILE=0|1 forces the choice (read at every call).
 static bool encode_use_wide(int N) {
   const char* e = getenv("LAPRUNE_ENCODE_TILE");

@@ -43,10 +43,10 @@
 // codebooks of trained magnitudes one entry is left for about 95 % of the
 // rows, and its distance need not be formed at all.
 //
-// Measured (1,048,576 rows, D = 128, trained magnitudes): 3.4 ms against 13.8
-// ms for the bf16 form it replaced (64 rows per workgroup, a barrier-separated
-// coarse pass, shortlist and recheck, 6.9 us per stage and 64 rows; here 6.4
-// us per 256).  What bounds it now is instruction issue: about 1120 VALU
+// Measured (1,048,576 rows, D = 128): 3.2 to 3.9 ms in six runs (3.3 to 3.6 with
+// entries of trained magnitudes) against 13.6 to 14.0 for the bf16 form it
+// replaced (64 rows per workgroup, a barrier-separated coarse pass, shortlist and
+// recheck, 6.9 us per stage and 64 rows; here 6.4 us per 256).  What bounds it now is instruction issue: about 1120 VALU
 // instructions per wave and stage (2.5 per score to find maximum and
 // survivors) fill some 60 % of the cycles and the products 33 %.
 #pragma once

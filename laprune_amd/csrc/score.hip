@@ -270,9 +270,9 @@ __global__ __launch_bounds__(THREADS) void score_g4p_kernel(
 // once and every lookup serves four heads; lanes of heads past G repeat head
 // G - 1 (a group maximum does not see them, and they are not written).  One
 // head per workgroup with two-byte lookups, which it replaced where the code
-// rows are aligned, read each code row G times and left the keys to a pass of
-// their own (G = 8, 4 x 65537 tokens: 27.4 us, here 12.3; G = 7, two sequences of
-// 4 x 50001 tokens: 2 x 22 and 18.5 us, here 12.9).  The lookups bound it: 64 per
+// rows are aligned and not few, read each code row G times and left the keys to a
+// pass of their own (G = 8, 4 x 65537 tokens: 27.4 us, here 12.4; G = 7, two
+// sequences of 4 x 50001 tokens: 2 x 22 and 18.5 us, here 13.0).  The lookups bound it: 64 per
 // token at G > 4, about six cycles per 64 lanes each, and the 128 KiB table fill
 // of every workgroup (about 2.5 us).  Outputs as
 // score_g4p_kernel: fp16 scores per head, or selection keys (group maximum, or

@@ -6,9 +6,9 @@ serves too: its scores come from the GQA gather kernel for any G
 window, budget and torch.topk (aq_evaluation.py:160-205).
 
 Head dim 256 (with G = 4, the fused scorer's chain) is covered here too.
-These shapes take the kernel chain: the per-head [B * Hq][32][256] table,
-lap_lut_score_gqa of every head, lap_topk_select (_ragged) over the group
-max (group selection) or each head's row, then the split-K sparse
+These shapes take the kernel chain: the per-head [B * Hq][32][256] table, one
+scorer for up to eight heads that writes the selection keys of the group max
+(group selection) or of each head, their top-k, then the split-K sparse
 attention.  Indices are checked bit for bit against the oracle's top-k of
 the oracle's scores and the attention within 1e-2 of float64 softmax over
 the keep set (:210-251), uniform and ragged, eager and from a replayed
