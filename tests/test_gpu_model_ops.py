@@ -254,6 +254,11 @@ def test_modes_and_traces_see_the_models_ops():
         assert c.get_total_flops() == 3 * 2 * 64 * 96
         traced = torch.jit.trace(lambda t: layer.mlp(t), x, check_trace=False)
         assert "laprune::" not in str(traced.graph)
+        from torch.fx.experimental.proxy_tensor import make_fx
+        graph = make_fx(lambda t: layer.mlp(t))(x).graph
+        assert not any("laprune" in str(n.target) for n in graph.nodes)
+        compiled = torch.compile(layer.mlp, backend="eager", fullgraph=True)
+        torch.testing.assert_close(compiled(x), layer.mlp(x), rtol=2 ** -6, atol=2 ** -9)
 
 
 def test_weights_of_another_class_keep_their_product():
